@@ -239,6 +239,25 @@ int luc_paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t 
                       int num_layers, int num_q_heads, int num_kv_heads, int head_dim,
                       int block_size, float sm_scale, void* out, int64_t out_row_stride);
 
+/* The same, with long contexts cut into K splits where the prompt rows alone
+ * would leave compute units idle: every split leaves f32 partials in
+ * `workspace` and a third launch merges them (outputs agree with
+ * luc_paged_prefill to f32 rounding of the sums).  The workspace holds at
+ * least luc_paged_prefill_workspace_size bytes of device memory, 256-byte
+ * aligned, contents arbitrary, used until the call's launches end; 0 (and
+ * NULL) means that these sizes need no split and the two calls are the same. */
+size_t luc_paged_prefill_workspace_size(int batch, int total_rows, int max_ctx, int num_q_heads,
+                                        int num_kv_heads, int head_dim);
+int luc_paged_prefill_split(luc_ctx* ctx, void* stream, int dtype, void* qkv,
+                            int64_t qkv_row_stride, const void* q_bias, const void* k_bias,
+                            const void* v_bias, const float* cos_table, const float* sin_table,
+                            void* k_pool, void* v_pool, const int32_t* block_tables,
+                            int table_stride, int num_blocks, const int32_t* cu_seqlens,
+                            const int32_t* start_pos, int batch, int total_rows, int max_ctx,
+                            int layer, int num_layers, int num_q_heads, int num_kv_heads,
+                            int head_dim, int block_size, float sm_scale, void* out,
+                            int64_t out_row_stride, void* workspace, size_t workspace_bytes);
+
 /* ---- The model loop's small kernels (bf16 only) ---- */
 
 /* RMSNorm of `rows` rows of `cols` elements: out = round((x * inv) * w) with

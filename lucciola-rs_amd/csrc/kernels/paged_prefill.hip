@@ -7,21 +7,28 @@
 // k and v + v_bias are in the cache (the append kernel, launched first on the
 // same stream).  q gets its bias and RoPE here, as each row's q is loaded
 // (the append kernel's arithmetic, bit for bit), and is written back in place
-// (when the tables allow 16-byte loads; else the append kernel ropes q too).  Row i of sequence b and q-head qh then attends to
+// (head_dim 64 with one split, and tables that allow 16-byte loads; else the
+// append kernel ropes q too).  Row i of sequence b and q-head qh then attends to
 // cache positions 0..start_pos[b] + i through table row b -- the cached prefix
 // and the prompt rows up to itself -- exactly what the reference's
 // flash_decoding call for that token computes (src/kernels/attention.cu:4-176),
 // since by then the cache holds those positions and nothing later.
 //
-// Work decomposition: workgroup = (sequence b, kv head h, pair p of tiles of
-// 32 prompt rows), one wave per q-head of the group of G = Hq/Hkv q-heads
-// (4 waves for G <= 4, else 8) over the same 32 rows, so the K and V tiles
-// staged in LDS serve every head of the group (GQA).  Of a sequence's nt row tiles the workgroup takes tile nt-1-p
-// and then tile p: causal tile t reads about t+1 token blocks, so every pair
-// carries the same work, the grid is one wave of equal workgroups and none
-// waits on a long tail.  For each tile the workgroup walks the tokens
-// 0..(last position of its rows) in blocks of 64, grouped into super-blocks
-// (two blocks at head_dim 64 with 8 waves, else one) in an LDS ring of NS
+// Work decomposition: the (prompt row, q-head of the group) pairs of a sequence
+// and kv head h, row-major (m = row * G + head, G = Hq / Hkv), in tiles of 32:
+// one tile per wave, chunks of 8 consecutive tiles per workgroup, so the K and
+// V tiles staged in LDS serve all heads of the group (GQA) and every wave has a
+// full tile at every G (also when the rows are few).  Workgroup = (K split s,
+// chunk c, sequence b, kv head h).  A split is a range of split_tokens
+// positions; the host cuts the contexts where the chunks alone leave CUs idle
+// (512 rows after 8000 cached, 12 q- and 2 kv-heads of 128: 24 chunks, 54 us a
+// call in 10 splits, 542 with every context in one workgroup of a head's rows).
+// Row i's position falls into the last split it reads: rows of positions below
+// split_tokens are finished by split 0, every other row's splits leave (max,
+// sum, unnormalised O) partials in the workspace for luc_prefill_merge.
+// Workgroups run longest first (split-major, the last chunk first), so short
+// ones fill the tail.  A workgroup walks its tokens in blocks of 64, grouped
+// into super-blocks (two blocks at head_dim 64, else one) in an LDS ring of NS
 // stages (four at head_dim 64, three at 128): super-block J + NS - 2 loads
 // while super-block J is computed, and the waves meet at one barrier per
 // super-block.
@@ -77,8 +84,14 @@ struct PrefillArgs {
   const uint16_t* q_bias;  // [Hq*D] or null
   const float* cos_t;      // [positions][D/2], 16-byte aligned, or null
   const float* sin_t;
-  int32_t batch, layer, num_layers, hkv, max_ctx, pairs;  // pairs: tile pairs per sequence
-  int32_t num_blocks;  // pages per pool: table entries outside [0, num_blocks) are never used
+  float* ws_ml;  // [splits][total_rows][Hq] (max, sum), with splits > 1
+  float* ws_o;   // [splits][total_rows][Hq][D]
+  int32_t batch, layer, num_layers, hkv, max_ctx;
+  int32_t chunks;        // workgroups per (split, sequence, kv head)
+  int32_t num_blocks;    // pages per pool: table entries outside [0, num_blocks) are never used
+  int32_t group;         // q-heads per kv head
+  int32_t split_tokens;  // positions per split, a multiple of 128 (>= max_ctx: one split)
+  int32_t total_rows;
   float qk_scale_log2;  // sm_scale * log2(e)
 };
 
@@ -210,21 +223,19 @@ __device__ constexpr uint32_t vslot(int t, int d) {
   return ((t >> 3) * (D / 32) + (d >> 5)) * 512 + ((t & 7) << 6) + (((d & 31) >> 2) << 3);
 }
 
-// Waves per prefill workgroup for group size G (<= 8): one per q-head.
-constexpr int prefill_waves(int g) { return g <= 4 ? 4 : 8; }
+constexpr int kPrefillWaves = 8;
 
-template <int DT, int D, int G>
+template <int DT, int D>
 __device__ void prefill_impl(const PrefillArgs& A) {
-  constexpr int W = prefill_waves(G);  // waves per workgroup: one per q-head of the group
-  constexpr int NHG = (G + W - 1) / W;
+  constexpr int W = kPrefillWaves;  // waves per workgroup: one 32-column tile each
   constexpr int BT = 64;          // tokens per block
   constexpr int CH = D / 8;       // 16-byte chunks per token row
   constexpr int ROWB = 2 * D;     // bytes per token row
   constexpr int KB = BT * ROWB;   // bytes of a K (or V) block
   // A stage holds SB consecutive blocks (a super-block): the waves meet at a
   // barrier once per stage.  Two blocks when the LDS of one workgroup per CU
-  // allows it (d64, 8 waves), else one.
-  constexpr int SB = (D == 64 && W == 8) ? 2 : 1;
+  // allows it (d64), else one.
+  constexpr int SB = D == 64 ? 2 : 1;
   constexpr int KS = SB * KB;     // bytes of the K (or V) part of a stage
   constexpr int LOADS = KS / 1024;       // 1 KB wave-wide loads per K (or V) part
   constexpr int TPL = 1024 / ROWB;       // tokens per 1 KB load
@@ -234,8 +245,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   // t at slot c ^ kkey(t); V at vslot): super-block j is loaded NS - 2 stages
   // before its scores
   constexpr int NS = D == 64 ? 4 : 3;
-  // head_dim 64 with two-block super-blocks (8 waves): the software-pipelined steps
-  constexpr bool PIPE = D == 64 && SB == 2;
+  constexpr bool PIPE = D == 64;  // the software-pipelined steps
   constexpr int LPW = 2 * LOADS / W;  // loads per wave per stage
   static_assert(LOADS % W == 0, "every wave issues the same number of K (and V) loads");
   __shared__ __attribute__((aligned(16))) char s_kv[NS][2][KS];
@@ -245,70 +255,96 @@ __device__ void prefill_impl(const PrefillArgs& A) {
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // pair-major order: every group's first pair is dispatched before any
-  // second pair, and consecutive workgroups (which the hardware spreads over
-  // the XCDs) belong to different groups
-  const int groups = A.batch * A.hkv * NHG;
-  const int pair = blockIdx.x / groups;
-  int rem = blockIdx.x - pair * groups;
-  const int b = rem / (A.hkv * NHG);
-  rem -= b * A.hkv * NHG;
-  const int h = rem / NHG;
-  const int hg = rem - h * NHG;
+  // split-major, then the last (longest) chunk first; consecutive workgroups
+  // (which the hardware spreads over the XCDs) belong to different (b, h)
+  const int G = A.group;
+  const int groups = A.batch * A.hkv;
+  int rem = blockIdx.x / groups;
+  const int bh = blockIdx.x - rem * groups;
+  const int split = rem / A.chunks;
+  const int chunk = A.chunks - 1 - (rem - split * A.chunks);
+  const int b = bh / A.hkv;
+  const int h = bh - b * A.hkv;
   const int row0 = A.cu_seqlens[b];
   const int nrows = A.cu_seqlens[b + 1] - row0;
   const int sp = A.start_pos[b];
-  const bool active = hg * W + w < G;  // wave-uniform: a q-head of the group
-  const int qh = h * G + min(hg * W + w, G - 1);
+  const int64_t ncols = (int64_t)nrows * G;  // (row, head) pairs of the sequence and kv head
   const int g = lane >> 5;
-  // q's RoPE here except in the 8-wave head_dim 128 kernels, which have no
-  // registers to spare (the host then has the append kernel rope q)
-  constexpr bool QROPE = !(D == 128 && W == 8);
-  // The lane's share of q-head row qrow (dims g*8 + 16k .. + 8, k < NK), with
-  // bias + RoPE at position pos: dims i and i + D/2 are pairs k and k + NK/2
-  // of the same lane.  Written back in place when `store`.
-  auto rope_q = [&](uint16_t* qrow, int pos, uint4* x, bool store) __attribute__((always_inline)) {
+  // q's RoPE here except at head_dim 128, where the kernel has no registers to
+  // spare (the host then has the append kernel rope q)
+  constexpr bool QROPE = D == 64;
+  // The lane's share of row qrow of q-head qh (dims g*8 + 16k .. + 8, k < NK)
+  // with its bias and the cos / sin of position pos: all loads, none waited
+  // for (a missing bias reads q in its place, masked to zero) ...
+  struct RopeIn {
+    uint4 x[NK], b[NK];
+    float4 c[NK], s[NK];  // (pairs of 4-float vectors per rotation unit)
+  };
+  const bool has_bias = A.q_bias != nullptr;
+  auto rope_load = [&](const uint16_t* qrow, int qh, int pos, RopeIn& r) __attribute__((always_inline)) {
+    const uint16_t* const brow = (has_bias ? A.q_bias + (int64_t)qh * D : qrow) + g * 8;
 #pragma unroll
-    for (int k = 0; k < NK; ++k) x[k] = *(const uint4*)(qrow + g * 8 + 16 * k);
-    const bool has_bias = A.q_bias != nullptr;
-    const uint16_t* const brow = A.q_bias + (int64_t)qh * D + g * 8;
+    for (int k = 0; k < NK; ++k) r.x[k] = *(const uint4*)(qrow + g * 8 + 16 * k);
 #pragma unroll
-    for (int k = 0; k < NK / 2; ++k) {
-      const uint4 zero = make_uint4(0, 0, 0, 0);
-      const uint4 b1 = has_bias ? *(const uint4*)(brow + 16 * k) : zero;
-      const uint4 b2 = has_bias ? *(const uint4*)(brow + 16 * k + D / 2) : zero;
-      const float4* cp = (const float4*)(A.cos_t + (int64_t)pos * (D / 2) + g * 8 + 16 * k);
-      const float4* spp = (const float4*)(A.sin_t + (int64_t)pos * (D / 2) + g * 8 + 16 * k);
-      rope_rotate8<DT>(x[k], x[k + NK / 2], b1, b2, has_bias, cp[0], cp[1], spp[0], spp[1]);
+    for (int k = 0; k < NK; ++k) r.b[k] = *(const uint4*)(brow + 16 * k);
+    const float* const cp = A.cos_t + (int64_t)pos * (D / 2) + g * 8;
+    const float* const np = A.sin_t + (int64_t)pos * (D / 2) + g * 8;
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      r.c[k] = *(const float4*)(cp + 16 * (k / 2) + 4 * (k % 2));
+      r.s[k] = *(const float4*)(np + 16 * (k / 2) + 4 * (k % 2));
     }
-    if (store)
+  };
+  // ... and the roped result: dims i and i + D/2 are pairs k and k + NK/2 of
+  // the same lane
+  auto rope_apply = [&](RopeIn& r, uint4* x) __attribute__((always_inline)) {
+    uint32_t bm = has_bias ? 0xffffffffu : 0u;
+    asm volatile("" : "+v"(bm));
 #pragma unroll
-      for (int k = 0; k < NK; ++k) *(uint4*)(qrow + g * 8 + 16 * k) = x[k];
+    for (int k = 0; k < NK; ++k) {
+      r.b[k] = make_uint4(r.b[k].x & bm, r.b[k].y & bm, r.b[k].z & bm, r.b[k].w & bm);
+      x[k] = r.x[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NK / 2; ++k)
+      rope_rotate8<DT>(x[k], x[k + NK / 2], r.b[k], r.b[k + NK / 2], true, r.c[2 * k], r.c[2 * k + 1],
+                       r.s[2 * k], r.s[2 * k + 1]);
   };
   if (sp < 0 || sp + nrows > A.max_ctx) {
     // positions outside the host bound: flagged with NaN, never truncated
-    // (such a sequence may have more tiles than the grid has pairs: the
-    // workgroups of its group stride over all its rows)
-    if (active)
-      for (int r = pair * 32 + (lane & 31); r < nrows; r += A.pairs * 32) {
-        uint16_t* const orow = A.out + (int64_t)(row0 + r) * A.out_stride + (int64_t)qh * D;
-        for (int d = 0; d < D; d += 8)
-          for (int j = 0; j < 4; ++j) orow[d + 4 * g + j] = St<DT>::store(__builtin_nanf(""));
-        // q still gets its RoPE where its position lies in the table row
-        const int64_t pos = (int64_t)sp + r;
-        if (QROPE && A.cos_t && pos >= 0 && pos < A.table_stride * kPage) {
-          uint4 qv[NK];
-          rope_q(A.qkv + (int64_t)(row0 + r) * A.qkv_stride + (int64_t)qh * D, (int)pos, qv, true);
-        }
+    // (such a sequence may have more columns than the grid has chunks: the
+    // workgroups of its split 0 stride over all of them)
+    if (split) return;
+    for (int64_t m = ((int64_t)chunk * W + w) * 32 + (lane & 31); m < ncols; m += (int64_t)A.chunks * W * 32) {
+      const int r = (int)(m / G);
+      const int qh = h * G + (int)(m - (int64_t)r * G);
+      uint16_t* const orow = A.out + (int64_t)(row0 + r) * A.out_stride + (int64_t)qh * D;
+      for (int d = 0; d < D; d += 8)
+        for (int j = 0; j < 4; ++j) orow[d + 4 * g + j] = St<DT>::store(__builtin_nanf(""));
+      // q still gets its RoPE where its position lies in the table row
+      const int64_t pos = (int64_t)sp + r;
+      if (QROPE && A.cos_t && pos >= 0 && pos < A.table_stride * kPage) {
+        RopeIn in;
+        uint4 qv[NK];
+        uint16_t* const qrow = A.qkv + (int64_t)(row0 + r) * A.qkv_stride + (int64_t)qh * D;
+        rope_load(qrow, qh, (int)pos, in);
+        rope_apply(in, qv);
+#pragma unroll
+        for (int k = 0; k < NK; ++k) *(uint4*)(qrow + g * 8 + 16 * k) = qv[k];
       }
+    }
     return;
   }
-  const int nt = (nrows + 31) / 32;  // row tiles of the sequence (nt <= 2 * pairs)
-  if (pair >= (nt + 1) / 2) return;
+  // within the bound: nrows <= max_ctx, and chunks covers its columns
+  if ((int64_t)chunk * (W * 32) >= ncols) return;
+  const int c0 = chunk * (W * 32);  // first column of the workgroup
+  const int last = sp + min((c0 + W * 32 - 1) / G, nrows - 1);  // last position of its rows
+  const int tok0 = split * A.split_tokens;
+  if (tok0 > last) return;
+  const int nkv = min(last + 1, tok0 + A.split_tokens);  // the split's tokens are tok0 .. nkv - 1
   const int* trow = A.tables + (int64_t)b * A.table_stride;
   const int64_t page_stride = (int64_t)A.num_layers * A.hkv * kPage * D;
   const int64_t head_off = ((int64_t)A.layer * A.hkv + h) * kPage * D;
-  const int ntiles = pair < nt - 1 - pair ? 2 : 1;
   // exponents are exp2(s * scale - max): with q negated for a negative scale
   // the scale is positive, so the row max of s * scale is (max s) * scale
   const bool neg_scale = A.qk_scale_log2 < 0.0f;
@@ -352,15 +388,20 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   uint32_t lane_off[LPW];
 #pragma unroll
   for (int i = 0; i < LPW; ++i) lane_off[i] = KEEP_OFF ? load_offset(i, load_token(i, lane) % kPage, lane) : 0;
-  for (int k = 0; k < ntiles; ++k) {
-  const int rt = k == 0 ? nt - 1 - pair : pair;
-  const int my_i = rt * 32 + (lane & 31);  // the lane's prompt row (q row of the tile)
-  const bool row_ok = active && my_i < nrows;
+  // the wave's 32 columns, one per lane pair (l, l + 32)
+  const int w0 = c0 + 32 * w;
+  const int my_m = w0 + (lane & 31);
+  const int my_i = min(my_m, (int)ncols - 1) / G;  // the lane's prompt row
+  const int qh = h * G + min(my_m, (int)ncols - 1) - my_i * G;  // and q-head
+  const bool row_ok = my_m < ncols;
   const int my_pos = sp + my_i;
-  uint16_t* const orow = A.out + (int64_t)(row0 + min(my_i, nrows - 1)) * A.out_stride + (int64_t)qh * D;
-  const int last = sp + min(rt * 32 + 32, nrows) - 1;  // last position of the tile's rows
-  const int nkv = last + 1;  // tokens the tile reads
-  const int nblk = (nkv + BT - 1) / BT;
+  const int first_pos = sp + min(w0, (int)ncols - 1) / G;  // first and last position of the wave's rows
+  const int last_pos = sp + min(w0 + 31, (int)ncols - 1) / G;
+  const bool active = w0 < ncols && last_pos >= tok0;  // wave-uniform
+  uint16_t* const orow = A.out + (int64_t)(row0 + my_i) * A.out_stride + (int64_t)qh * D;
+  const int nblk = (nkv - tok0 + BT - 1) / BT;
+  // blocks that the wave's own rows reach
+  const int wblk = active ? min(nblk, (last_pos - tok0) / BT + 1) : 0;
 
   // Page numbers of super-block sb that this wave's loads need: load jj
   // covers TPL tokens of one page (TPL divides the page), jj = i * W + w for
@@ -368,7 +409,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   // scalar cache, read a stage before the loads they address and checked
   // only there, so their round trip overlaps a block's compute.
   constexpr int NPG = LOADS / W;
-  auto page_index = [&](int sb, int i) { return min(sb * SB * BT + (i * W + w) * TPL, nkv - 1) / kPage; };
+  auto page_index = [&](int sb, int i) { return min(tok0 + sb * SB * BT + (i * W + w) * TPL, nkv - 1) / kPage; };
   auto load_pages = [&](int sb, int* pg) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NPG; ++i) pg[i] = ((const const_i32_p*)trow)[page_index(sb, i)];
@@ -389,7 +430,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
       if (!ok) bad_tok = min(bad_tok, page_index(sb, i) * kPage);
       pv[i] = ok ? pg[i] : 0;
     }
-    const int sbase = sb * SB * BT;
+    const int sbase = tok0 + sb * SB * BT;
     // uniform: every token of the stage inside the context, so every lane
     // reads at its fixed offset within the page (a 32-bit offset from the
     // page row's scalar base address)
@@ -420,21 +461,30 @@ __device__ void prefill_impl(const PrefillArgs& A) {
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
   static_assert(NS - 2 <= 2, "wait_blocks covers up to two newer super-blocks");
-  // Q^T fragments (B operand): lane l holds q row my_i, dims (l/32)*8 + 16k .. +8
-  // (loaded before the tile's first K/V loads are issued, so the block waits
-  // below count only block loads)
-  // (with q's RoPE here, loaded and roped once the tile's first super-block
-  // of K/V loads is issued: the two latencies overlap, and that super-block
-  // is waited for before the first scores anyway; written back at the tile's
-  // end)
+  // Q^T fragments (B operand): lane l holds q row my_i, dims (l/32)*8 + 16k .. +8.
+  // All loads of q and its RoPE go out here, before the table entries that
+  // the K/V loads wait for have arrived; roped once the first K/V loads are
+  // issued (the latencies overlap, and those are waited for before the first
+  // scores anyway); written back at the end.  With these loads, and all of the
+  // prologue's table entries, in one round trip each, a workgroup's prologue takes
+  // 5.0 us; with the bias and cos / sin loads behind a branch and the K/V loads, and
+  // the entries read where they are used, 8.3 (timestamps; head_dim 64, 14 q- and
+  // 2 kv-heads, 4 x 2048 rows).
   uint4 qf[NK];
-  uint16_t* const qrow = A.qkv + (int64_t)(row0 + min(my_i, nrows - 1)) * A.qkv_stride + (int64_t)qh * D;
+  uint16_t* const qrow = A.qkv + (int64_t)(row0 + my_i) * A.qkv_stride + (int64_t)qh * D;
   const bool qrope = QROPE && A.cos_t != nullptr;  // wave-uniform
-  if (!qrope)
+  RopeIn rin;
+  if (qrope)
+    rope_load(qrow, qh, my_pos, rin);
+  else
 #pragma unroll
-    for (int k = 0; k < NK; ++k) qf[k] = *(const uint4*)(qrow + g * 8 + 16 * k);
+    for (int k = 0; k < NK; ++k) rin.x[k] = *(const uint4*)(qrow + g * 8 + 16 * k);
   auto finish_q = [&]() __attribute__((always_inline)) {
-    if (qrope) rope_q(qrow, sp + min(my_i, nrows - 1), qf, false);
+    if (qrope)
+      rope_apply(rin, qf);
+    else
+#pragma unroll
+      for (int k = 0; k < NK; ++k) qf[k] = rin.x[k];
     if (neg_scale)  // S = -(K Q^T) exactly: sign flips commute with rounding
 #pragma unroll
       for (int k = 0; k < NK; ++k) {
@@ -474,7 +524,8 @@ __device__ void prefill_impl(const PrefillArgs& A) {
     for (int e = 0; e < 16; ++e) o[i][e] = 0.0f;
 #pragma unroll
   for (int e = 0; e < 16; ++e) osum[e] = 0.0f;
-  float m_run = -INFINITY;
+  // (finite, so that a row whose first blocks are all masked keeps zero sums)
+  float m_run = -3.402823466e38f;
   // all-ones A operand: its MFMA with P^T sums P over the block's tokens
   const uint32_t one2 = DT == kF16 ? 0x3c003c00u : 0x3f803f80u;
   const uint4 ones = make_uint4(one2, one2, one2, one2);
@@ -490,7 +541,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
     // lazy running max: it moves only when some row's block max passes it by
     // more than kLazyMax (then every row takes its new max), so exponents
     // stay below 2^kLazyMax and the rescale of o is rare
-    const float m_blk = mb * scale;  // finite: token 0 is in every row's range
+    const float m_blk = mb * scale;
     if (__builtin_amdgcn_ballot_w64(m_blk > m_run + kLazyMax) != 0) {  // wave-uniform
       const float m_new = fmaxf(m_run, m_blk);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -504,9 +555,9 @@ __device__ void prefill_impl(const PrefillArgs& A) {
     }
   };
   // block blk entirely at or before the tile's first row position: no mask
-  auto unmasked = [&](int blk) { return blk * BT + BT - 1 <= sp + rt * 32; };
+  auto unmasked = [&](int blk) { return tok0 + blk * BT + BT - 1 <= first_pos; };
   auto softmax_max = [&](int blk, f32x16* sc) __attribute__((always_inline)) {
-    const int t0 = blk * BT;
+    const int t0 = tok0 + blk * BT;
     // sc[hf][4i + j]: token t0 + 32hf + 8i + 4g + j, q row my_i
     float mb = -INFINITY;
     if (unmasked(blk)) {  // wave-uniform: below the diagonal
@@ -583,91 +634,42 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   // and the barrier also tells every wave that super-block J-2 is consumed,
   // so its stage takes super-block J + NS - 2.
   const int nsb = (nblk + SB - 1) / SB;
-  auto boundary = [&](int blk, bool prefetch) __attribute__((always_inline)) {  // before block blk + 1
+  auto boundary = [&](int blk) __attribute__((always_inline)) {  // before block blk + 1
     if ((blk + 1) % SB == 0) {
       const int J = (blk + 1) / SB;
       wait_blocks(min(NS - 3, nsb - 1 - J));
       __builtin_amdgcn_s_barrier();
       if (J + NS - 2 < nsb) {
         issue(J + NS - 2, (J + NS - 2) % NS, pgn);
-        if (prefetch && J + NS - 1 < nsb) load_pages(J + NS - 1, pgn);
+        if (J + NS - 1 < nsb) load_pages(J + NS - 1, pgn);
       }
-    }
-  };
-  // the table entries the next boundary issues from, read once this block's
-  // work is issued (head_dim 64)
-  auto prefetch_pages = [&](int blk) __attribute__((always_inline)) {
-    if ((blk + 1) % SB == 0) {
-      const int J = (blk + 1) / SB;
-      if (J + NS - 1 < nsb) load_pages(J + NS - 1, pgn);
     }
   };
   auto step = [&](int blk, f32x16* cur, f32x16* nxt) __attribute__((always_inline)) {
-    if constexpr (D == 64) {
-      // the LDS reads of K(blk + 1) and of the first half of V(blk) go out
-      // before the mask and max of block blk, the second half of V(blk)
-      // before its exponentials, so they land while the VALU works; the
-      // scores of blk + 1 reach the matrix cores before the exponentials,
-      // the PV of blk after them
-      u32x4_t ka[8];
-      u32x2_t va[16];
-      const bool has_next = blk + 1 < nblk;
-      if (has_next) {
-        boundary(blk, false);
-        if (active) {
-          const uint32_t kbase = lds_addr(s_kv[((blk + 1) / SB) % NS][0]) + ((blk + 1) % SB) * KB;
-          lds_k_issue<32 * ROWB>(kbase + krel[0], kbase + krel[1], kbase + krel[2], kbase + krel[3], ka);
-        }
-      }
-      if (active) {
-        const uint32_t vbase = lds_addr(s_kv[(blk / SB) % NS][1]) + (blk % SB) * KB;
-        lds_v_issue_half<ROWB, 0>(vbase + vrel[0], vbase + vrel[1], va);
-        softmax_max(blk, cur);
-        if (has_next) {
-          lds_wait_k<8>(ka);  // the first V reads of this block may still be in flight
-#pragma unroll
-          for (int hf = 0; hf < 2; ++hf) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) nxt[hf][e] = 0.0f;
-#pragma unroll
-            for (int k = 0; k < NK; ++k)
-              nxt[hf] = mfma32<DT>(__builtin_bit_cast(uint4, ka[4 * hf + k]), qf[k], nxt[hf]);
-          }
-        }
-        lds_v_issue_half<ROWB, 1>(vbase + vrel[0], vbase + vrel[1], va);
-        softmax_exp(cur);
-        lds_wait_v(va);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const uint4 pb = p_operand(cur, c >> 1, c & 1);
-          osum = mfma32<DT>(ones, pb, osum);
-#pragma unroll
-          for (int db = 0; db < ND; ++db)
-            o[db] = mfma32<DT>(make_uint4(va[4 * c + 2 * db].x, va[4 * c + 2 * db].y,
-                                          va[4 * c + 2 * db + 1].x, va[4 * c + 2 * db + 1].y),
-                               pb, o[db]);
-        }
-      }
-      if (has_next) prefetch_pages(blk);
-    } else {
-      if (blk + 1 < nblk) {
-        boundary(blk, true);
-        if (active) qk(blk + 1, nxt);
-      }
-      if (active) softmax_pv(blk, cur);
+    if (blk + 1 < nblk) {
+      boundary(blk);
+      if (blk + 1 < wblk) qk(blk + 1, nxt);
     }
+    if (blk < wblk) softmax_pv(blk, cur);
   };
 
-  // every wave is done with the previous tile's last stage before it is refilled
-  if (k) __builtin_amdgcn_s_barrier();
   if (threadIdx.x == 0) s_bad_tok = 0x7fffffff;  // (read by every wave only after a barrier below)
+  {
+    // the table entries of every super-block issued here in one round trip
+    // (clamped to the context; pinned, or the compiler would load each where
+    // it is used)
+    int pg[NS - 1][NPG];
 #pragma unroll
-  for (int j = 0; j < NS - 1; ++j) {
-    if (j < nsb) {
-      load_pages(j, pgn);
-      issue(j, j, pgn);
-    }
-    if (j == 0) finish_q();  // (q's loads and super-block 0's are in flight together)
+    for (int j = 0; j < NS - 1; ++j) load_pages(j, pg[j]);
+#pragma unroll
+    for (int j = 0; j < NS - 1; ++j)
+#pragma unroll
+      for (int i = 0; i < NPG; ++i) asm volatile("" : "+s"(pg[j][i]));
+    issue(0, 0, pg[0]);
+    finish_q();  // (q's loads and super-block 0's are in flight together)
+#pragma unroll
+    for (int j = 1; j < NS - 1; ++j)
+      if (j < nsb) issue(j, j, pg[j]);
   }
   if (NS - 1 < nsb) load_pages(NS - 1, pgn);
   wait_blocks(min(NS - 2, nsb - 1));
@@ -741,7 +743,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
           }
         }
       }
-      if (!active) return;
+      if (blk >= wblk) return;
       // K(blk + 1), both halves; V(blk), issued after them, may be in flight
       lds_wait_k<15>(ka);
       float mx[2] = {-INFINITY, -INFINITY};
@@ -790,10 +792,10 @@ __device__ void prefill_impl(const PrefillArgs& A) {
       // compiler would move it behind that branch, out of the MFMA shadow)
       asm volatile("" ::"v"(mx[0]), "v"(mx[1]));
       read_v(blk + 1);  // (past the last block: read, never used)
-      if (blk + 1 < nblk) {  // wave-uniform
+      if (blk + 1 < wblk) {  // wave-uniform
         float mb = fmaxf(mx[0], mx[1]);
         if (!unmasked(blk + 1)) {  // mask the diagonal block, its max again
-          const int t0 = (blk + 1) * BT;
+          const int t0 = tok0 + (blk + 1) * BT;
           mb = -INFINITY;
 #pragma unroll
           for (int hf = 0; hf < 2; ++hf)
@@ -842,20 +844,22 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   if (lane == 0 && bad_tok != 0x7fffffff) atomicMin(&s_bad_tok, bad_tok);
   __syncthreads();
   const int first_bad = s_bad_tok;
-  if (!active) continue;
-  if (row_ok) {
-    if (qrope)  // the roped q, in place (its sign flip undone); stored here, not
-                // in the prologue, so that no wait for the tile's first loads
-                // waits for these stores too
+  if (!active || !row_ok || my_pos < tok0) return;  // (a row below the split: none of its tokens)
+  if (qrope) {  // the roped q, in place (its sign flip undone); stored here, not
+                // in the prologue, so that no wait for the first loads waits
+                // for these stores too
 #pragma unroll
-      for (int k = 0; k < NK; ++k) {
-        uint4 x = qf[k];
-        if (neg_scale) {
-          x.x ^= 0x80008000u; x.y ^= 0x80008000u; x.z ^= 0x80008000u; x.w ^= 0x80008000u;
-        }
-        *(uint4*)(qrow + g * 8 + 16 * k) = x;
+    for (int k = 0; k < NK; ++k) {
+      uint4 x = qf[k];
+      if (neg_scale) {
+        x.x ^= 0x80008000u; x.y ^= 0x80008000u; x.z ^= 0x80008000u; x.w ^= 0x80008000u;
       }
-    const float inv = my_pos >= first_bad ? __builtin_nanf("") : 1.0f / osum[0];
+      *(uint4*)(qrow + g * 8 + 16 * k) = x;
+    }
+  }
+  const bool bad = my_pos >= first_bad;
+  if (my_pos < A.split_tokens) {  // (split 0, all of the row's context)
+    const float inv = bad ? __builtin_nanf("") : 1.0f / osum[0];
 #pragma unroll
     for (int db = 0; db < ND; ++db)
 #pragma unroll
@@ -864,28 +868,92 @@ __device__ void prefill_impl(const PrefillArgs& A) {
                                    pack2(o[db][4 * i + 2] * inv, o[db][4 * i + 3] * inv, DT));
         *(uint2*)(orow + db * 32 + 8 * i + 4 * g) = v;
       }
+  } else if (row0 + my_i < A.total_rows) {
+    const int64_t slot = ((int64_t)split * A.total_rows + row0 + my_i) * (A.hkv * G) + qh;
+    if (g == 0) *(float2*)(A.ws_ml + 2 * slot) = make_float2(m_run, bad ? __builtin_nanf("") : osum[0]);
+    float* const po = A.ws_o + slot * D + 4 * g;
+#pragma unroll
+    for (int db = 0; db < ND; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *(float4*)(po + db * 32 + 8 * i) =
+            make_float4(o[db][4 * i], o[db][4 * i + 1], o[db][4 * i + 2], o[db][4 * i + 3]);
   }
-  }  // tiles
+}
+
+// The rows whose contexts were cut: out = sum_s w_s O_s / sum_s w_s l_s with
+// w_s = exp2(m_s - max m), over splits 0 .. pos / split_tokens of the row.  D / 4
+// lanes per (packed row, q-head), four dims each.
+constexpr int kMergeThreads = 256;
+template <int DT, int D>
+__device__ void prefill_merge_impl(const PrefillArgs& A) {
+  constexpr int LPR = D / 4;  // lanes per (row, head)
+  const int hq = A.hkv * A.group;
+  const int64_t item = (int64_t)blockIdx.x * (kMergeThreads / LPR) + threadIdx.x / LPR;
+  if (item >= (int64_t)A.total_rows * hq) return;
+  const int r = (int)(item / hq);
+  const int qh = (int)(item - (int64_t)r * hq);
+  int lo = 0, hi = A.batch;  // the sequence of packed row r: cu_seqlens[lo] <= r < cu_seqlens[lo + 1]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (A.cu_seqlens[mid] <= r) lo = mid;
+    else hi = mid;
+  }
+  const int row0 = A.cu_seqlens[lo], nrows = A.cu_seqlens[lo + 1] - row0, sp = A.start_pos[lo];
+  if (r < row0 || r - row0 >= nrows || sp < 0 || sp + nrows > A.max_ctx) return;  // (the last: all NaN)
+  const int pos = sp + r - row0;
+  if (pos < A.split_tokens) return;  // written by split 0
+  const int ns = pos / A.split_tokens + 1;
+  const int64_t stride = (int64_t)A.total_rows * hq;  // slots from split to split
+  const float2* const ml = (const float2*)A.ws_ml + item;
+  const float* const po = A.ws_o + item * D + 4 * (threadIdx.x % LPR);
+  constexpr int U = 4;  // partials in flight
+  float m = -3.402823466e38f, l = 0.0f;
+  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int s0 = 0; s0 < ns; s0 += U) {
+    float2 x[U];
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t s = min(s0 + u, ns - 1);
+      x[u] = ml[s * stride];
+      v[u] = *(const float4*)(po + s * stride * D);
+    }
+    float mn = m;
+#pragma unroll
+    for (int u = 0; u < U; ++u) mn = fmaxf(mn, x[u].x);
+    const float a = __builtin_amdgcn_exp2f(m - mn);
+    m = mn;
+    l *= a;
+    acc.x *= a; acc.y *= a; acc.z *= a; acc.w *= a;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s0 + u >= ns) break;
+      const float wt = __builtin_amdgcn_exp2f(x[u].x - m);
+      l = fmaf(wt, x[u].y, l);
+      acc.x = fmaf(wt, v[u].x, acc.x);
+      acc.y = fmaf(wt, v[u].y, acc.y);
+      acc.z = fmaf(wt, v[u].z, acc.z);
+      acc.w = fmaf(wt, v[u].w, acc.w);
+    }
+  }
+  const float inv = 1.0f / l;
+  *(uint2*)(A.out + (int64_t)r * A.out_stride + (int64_t)qh * D + 4 * (threadIdx.x % LPR)) =
+      make_uint2(pack2(acc.x * inv, acc.y * inv, DT), pack2(acc.z * inv, acc.w * inv, DT));
 }
 
 }  // namespace luc
 
-#define LUC_PREFILL(DTN, DT, D, G)                                                              \
-  extern "C" __global__ __launch_bounds__(64 * luc::prefill_waves(G)) void luc_prefill_##DTN##_d##D##_g##G(             \
+#define LUC_PREFILL(DTN, DT, D)                                                                 \
+  extern "C" __global__ __launch_bounds__(64 * luc::kPrefillWaves) void luc_prefill_##DTN##_d##D(    \
       luc::PrefillArgs a) {                                                                     \
-    luc::prefill_impl<DT, D, G>(a);                                                             \
+    luc::prefill_impl<DT, D>(a);                                                                \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(luc::kMergeThreads) void luc_prefill_merge_##DTN##_d##D(   \
+      luc::PrefillArgs a) {                                                                     \
+    luc::prefill_merge_impl<DT, D>(a);                                                          \
   }
-#define LUC_PREFILL_GROUPS(DTN, DT, D)                                                          \
-  LUC_PREFILL(DTN, DT, D, 1)                                                                    \
-  LUC_PREFILL(DTN, DT, D, 2)                                                                    \
-  LUC_PREFILL(DTN, DT, D, 3)                                                                    \
-  LUC_PREFILL(DTN, DT, D, 4)                                                                    \
-  LUC_PREFILL(DTN, DT, D, 5)                                                                    \
-  LUC_PREFILL(DTN, DT, D, 6)                                                                    \
-  LUC_PREFILL(DTN, DT, D, 7)                                                                    \
-  LUC_PREFILL(DTN, DT, D, 8)
-
-LUC_PREFILL_GROUPS(bf16, luc::kBF16, 64)
-LUC_PREFILL_GROUPS(bf16, luc::kBF16, 128)
-LUC_PREFILL_GROUPS(f16, luc::kF16, 64)
-LUC_PREFILL_GROUPS(f16, luc::kF16, 128)
+LUC_PREFILL(bf16, luc::kBF16, 64)
+LUC_PREFILL(bf16, luc::kBF16, 128)
+LUC_PREFILL(f16, luc::kF16, 64)
+LUC_PREFILL(f16, luc::kF16, 128)

@@ -402,9 +402,76 @@ struct PrefillArgs {
   const void* q_bias;
   const float* cos_t;
   const float* sin_t;
-  int32_t batch, layer, num_layers, hkv, max_ctx, pairs, num_blocks;
+  float* ws_ml;
+  float* ws_o;
+  int32_t batch, layer, num_layers, hkv, max_ctx, chunks, num_blocks, group, split_tokens, total_rows;
   float qk_scale_log2;
 };
+
+// Prefill work split.  A workgroup takes a chunk of 256 (row, head of the
+// group) columns of one (sequence, kv head) and one K split.  With fewer
+// chunks than CUs, the contexts are cut into splits of `tokens` positions
+// (a multiple of 128) so that the grid fills the chip.  The lengths are on the device;
+// the plan takes `batch` sequences of equal rows that end at max_ctx, which
+// for one sequence is exact.  Cost in 64-token blocks: a workgroup takes its
+// blocks plus kPrefillUnit (prologue, epilogue, partials); the launch, its
+// longest workgroup or, with more than a round of them, the mean load of a CU
+// plus half a workgroup of tail.  Depends only on the arguments.
+constexpr int kPrefillCols = 256;    // columns per workgroup: 8 waves x 32 (paged_prefill.hip)
+struct PrefillPlan {
+  int chunks = 0;  // per (sequence, kv head), at most
+  int splits = 1;
+  int tokens = INT32_MAX;
+};
+constexpr int kPrefillSlots = kCUs;  // resident workgroups: one per CU
+constexpr int kPrefillUnit = 4;      // blocks
+constexpr int kPrefillMerge = 4;     // blocks: q's RoPE in the append kernel, the merge launch
+constexpr int kMaxPrefillSplits = 64;
+PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_ctx) {
+  PrefillPlan p;
+  const int64_t rows = std::min(total_rows, max_ctx);
+  p.chunks = (int)ceil_div(rows * group, kPrefillCols);
+  const int64_t seq_rows = std::min<int64_t>(rows, ceil_div(total_rows, batch));
+  const int64_t n = ceil_div(seq_rows * group, kPrefillCols);  // chunks of a mean sequence
+  const int64_t groups = (int64_t)batch * hkv;
+  if (n * groups >= kPrefillSlots || max_ctx > (1 << 28)) return p;
+  const int64_t prefix = std::max<int64_t>(max_ctx - seq_rows, 0);
+  int64_t best = INT64_MAX;
+  int64_t last_tokens = 0;
+  for (int s = 1; s <= kMaxPrefillSplits; s += s < 16 ? 1 : 4) {
+    const int64_t tokens = ceil_div(ceil_div(max_ctx, s), 128) * 128;
+    if (tokens == last_tokens) continue;
+    last_tokens = tokens;
+    int64_t units = 0, blocks = 0;
+    for (int64_t c = 0; c < n; ++c) {
+      const int64_t ctx = prefix + std::min(seq_rows, ceil_div((c + 1) * kPrefillCols, group));
+      units += ceil_div(ctx, tokens);
+      blocks += ceil_div(ctx, 64);
+    }
+    units *= groups;
+    blocks *= groups;
+    const int64_t unit = std::min<int64_t>(tokens, max_ctx) / 64 + kPrefillUnit;
+    // in 1 / kPrefillSlots of a block
+    int64_t cost = unit * kPrefillSlots;
+    if (units > kPrefillSlots) cost = std::max(cost, blocks + kPrefillUnit * units + unit * kPrefillSlots / 2);
+    if (s > 1) cost += kPrefillMerge * kPrefillSlots;
+    if (cost < best) {
+      best = cost;
+      p.splits = (int)ceil_div(max_ctx, tokens);
+      p.tokens = p.splits > 1 ? (int)tokens : INT32_MAX;
+    }
+  }
+  return p;
+}
+
+// Partials of a split launch: (max, sum) and o per (split, packed row, q-head), f32.
+size_t prefill_ml_bytes(const PrefillPlan& p, int total_rows, int hq) {
+  return align256((int64_t)p.splits * total_rows * hq * 2 * 4);
+}
+size_t prefill_workspace_bytes(const PrefillPlan& p, int total_rows, int hq, int head_dim) {
+  if (p.splits <= 1) return 0;
+  return prefill_ml_bytes(p, total_rows, hq) + (size_t)p.splits * total_rows * hq * head_dim * 4;
+}
 
 int launch_decode(DecodeLaunch& L, void* stream) {
   void* args[] = {&L.a};
@@ -468,9 +535,8 @@ int luc_init(int device, const char* code_object_dir, luc_ctx** out_ctx) {
     names.push_back(std::string("luc_rope_append_") + dt);
     for (int d : {64, 128}) names.push_back(std::string("luc_rope_append_vec_") + dt + "_d" + std::to_string(d));
     for (int d : {64, 128})
-      for (int g = 1; g <= 8; ++g)
-        names.push_back(std::string("luc_prefill_") + dt + "_d" + std::to_string(d) + "_g" +
-                        std::to_string(g));
+      for (const char* kind : {"luc_prefill_", "luc_prefill_merge_"})
+        names.push_back(std::string(kind) + dt + "_d" + std::to_string(d));
     for (int d : {64, 128})
       for (int g = 1; g <= 8; ++g)
         for (const char* kind : {"luc_decode_", "luc_decode_step_"}) {
@@ -683,14 +749,15 @@ int luc_decode_step_noalloc(luc_ctx* ctx, void* stream, int dtype, void* qkv,
                          ctx->scratch, LUC_SCRATCH_BYTES);
 }
 
-int luc_paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t qkv_row_stride,
+static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t qkv_row_stride,
                       const void* q_bias, const void* k_bias, const void* v_bias,
                       const float* cos_table, const float* sin_table, void* k_pool, void* v_pool,
                       const int32_t* block_tables, int table_stride, int num_blocks,
                       const int32_t* cu_seqlens,
                       const int32_t* start_pos, int batch, int total_rows, int max_ctx, int layer,
                       int num_layers, int num_q_heads, int num_kv_heads, int head_dim,
-                      int block_size, float sm_scale, void* out, int64_t out_row_stride) {
+                         int block_size, float sm_scale, void* out, int64_t out_row_stride,
+                         bool split, void* workspace, size_t workspace_bytes) {
   if (int rc = check_common(ctx, dtype, head_dim)) return rc;
   if (int rc = check_heads(num_q_heads, num_kv_heads)) return rc;
   if (int rc = check_cache(k_pool, v_pool, block_tables, table_stride, num_blocks, layer,
@@ -711,28 +778,30 @@ int luc_paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t 
   if ((int64_t)table_stride * LUC_BLOCK_SIZE < max_ctx)
     return fail(LUC_E_INVALID, "table_stride %d pages cannot hold max_ctx %d", table_stride, max_ctx);
   if (batch == 0 || total_rows == 0) return LUC_OK;
-  if (int rc = check_device(ctx)) return rc;
   const int group = num_q_heads / num_kv_heads;
-  hipFunction_t fn;
-  if (int rc = get_fn(ctx, std::string("luc_prefill_") + dt_name(dtype) + "_d" +
-                               std::to_string(head_dim) + "_g" + std::to_string(group),
-                      &fn))
-    return rc;
-  // workgroups: (sequence, kv head, pair of 32-row tiles), one wave per
-  // q-head of the group.  A sequence within the bound has at most
-  // min(total_rows, max_ctx) rows, so row_tiles tiles of 32 rows
-  const int row_tiles = (int)ceil_div(std::min(total_rows, max_ctx), 32);
-  const int pairs = (int)ceil_div(row_tiles, 2);
-  const int waves = group <= 4 ? 4 : 8;  // one per q-head of the group (paged_prefill.hip)
-  const int64_t grid = (int64_t)batch * num_kv_heads * ceil_div(group, waves) * pairs;
+  PrefillPlan plan = prefill_plan(batch, num_kv_heads, group, total_rows, max_ctx);
+  if (!split) {
+    plan.splits = 1;
+    plan.tokens = INT32_MAX;
+  }
+  const size_t need = prefill_workspace_bytes(plan, total_rows, num_q_heads, head_dim);
+  if (need && (!workspace || workspace_bytes < need))
+    return fail(LUC_E_WORKSPACE, "workspace %zu bytes, %zu needed", workspace_bytes, need);
+  if (need && !aligned(workspace, 256)) return fail(LUC_E_INVALID, "workspace must be 256-byte aligned");
+  if (int rc = check_device(ctx)) return rc;
+  const std::string suffix = std::string(dt_name(dtype)) + "_d" + std::to_string(head_dim);
+  hipFunction_t fn, merge;
+  if (int rc = get_fn(ctx, "luc_prefill_" + suffix, &fn)) return rc;
+  if (int rc = get_fn(ctx, "luc_prefill_merge_" + suffix, &merge)) return rc;
+  const int64_t grid = (int64_t)batch * num_kv_heads * plan.chunks * plan.splits;
   if (grid > INT32_MAX) return fail(LUC_E_INVALID, "batch x kv heads x row tiles too large");
 
   // q's bias + RoPE runs in the attention kernel, which loads every row's q
-  // anyway, when the bias and the rotation tables allow its 16-byte loads
-  // (not in the 8-wave head_dim 128 kernels: paged_prefill.hip, QROPE); else
-  // the append kernel ropes q as well
+  // anyway, when the bias and the rotation tables allow its 16-byte loads and
+  // one workgroup alone reads a row (no splits); not at head_dim 128
+  // (paged_prefill.hip, QROPE); else the append kernel ropes q as well
   const bool fuse_q = (!q_bias || aligned(q_bias, 16)) && aligned(cos_table, 16) &&
-                      aligned(sin_table, 16) && !(head_dim == 128 && group > 4);
+                      aligned(sin_table, 16) && head_dim == 64 && plan.splits == 1;
   // 1) bias + RoPE of every prompt row's k (and q unless fused) in place,
   //    cache write of the roped k and v + v_bias (models.rs:505-534 for each row)
   uint16_t* base = static_cast<uint16_t*>(qkv);
@@ -754,10 +823,60 @@ int luc_paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t 
   p.start_pos = start_pos; p.out = out; p.out_stride = out_row_stride; p.batch = batch;
   p.q_bias = q_bias; p.cos_t = fuse_q ? cos_table : nullptr; p.sin_t = sin_table;
   p.layer = layer; p.num_layers = num_layers; p.hkv = num_kv_heads; p.max_ctx = max_ctx;
-  p.pairs = pairs; p.num_blocks = num_blocks; p.qk_scale_log2 = sm_scale * 1.4426950408889634f;
+  p.chunks = plan.chunks; p.num_blocks = num_blocks; p.group = group; p.split_tokens = plan.tokens;
+  p.total_rows = total_rows; p.qk_scale_log2 = sm_scale * 1.4426950408889634f;
+  if (need) {
+    p.ws_ml = static_cast<float*>(workspace);
+    p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) +
+                                      prefill_ml_bytes(plan, total_rows, num_q_heads));
+  }
   void* args[] = {&p};
-  return launch(fn, dim3((unsigned)grid), dim3(64 * waves), stream, args);
+  if (int rc = launch(fn, dim3((unsigned)grid), dim3(2 * kPrefillCols), stream, args)) return rc;
+  if (!need) return LUC_OK;
+  // 3) the rows that several splits share (head_dim / 4 lanes per row and head)
+  const int64_t items = (int64_t)total_rows * num_q_heads;
+  return launch(merge, dim3((unsigned)ceil_div(items, 1024 / head_dim)), dim3(256), stream, args);
 }
+
+int luc_paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t qkv_row_stride,
+                      const void* q_bias, const void* k_bias, const void* v_bias,
+                      const float* cos_table, const float* sin_table, void* k_pool, void* v_pool,
+                      const int32_t* block_tables, int table_stride, int num_blocks,
+                      const int32_t* cu_seqlens, const int32_t* start_pos, int batch, int total_rows,
+                      int max_ctx, int layer, int num_layers, int num_q_heads, int num_kv_heads,
+                      int head_dim, int block_size, float sm_scale, void* out, int64_t out_row_stride) {
+  return paged_prefill(ctx, stream, dtype, qkv, qkv_row_stride, q_bias, k_bias, v_bias, cos_table,
+                       sin_table, k_pool, v_pool, block_tables, table_stride, num_blocks, cu_seqlens,
+                       start_pos, batch, total_rows, max_ctx, layer, num_layers, num_q_heads,
+                       num_kv_heads, head_dim, block_size, sm_scale, out, out_row_stride, false,
+                       nullptr, 0);
+}
+
+size_t luc_paged_prefill_workspace_size(int batch, int total_rows, int max_ctx, int num_q_heads,
+                                        int num_kv_heads, int head_dim) {
+  if (batch <= 0 || total_rows <= 0 || max_ctx <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 ||
+      num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > 8 || (head_dim != 64 && head_dim != 128))
+    return 0;
+  return prefill_workspace_bytes(
+      prefill_plan(batch, num_kv_heads, num_q_heads / num_kv_heads, total_rows, max_ctx), total_rows,
+      num_q_heads, head_dim);
+}
+
+int luc_paged_prefill_split(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t qkv_row_stride,
+                            const void* q_bias, const void* k_bias, const void* v_bias,
+                            const float* cos_table, const float* sin_table, void* k_pool, void* v_pool,
+                            const int32_t* block_tables, int table_stride, int num_blocks,
+                            const int32_t* cu_seqlens, const int32_t* start_pos, int batch,
+                            int total_rows, int max_ctx, int layer, int num_layers, int num_q_heads,
+                            int num_kv_heads, int head_dim, int block_size, float sm_scale, void* out,
+                            int64_t out_row_stride, void* workspace, size_t workspace_bytes) {
+  return paged_prefill(ctx, stream, dtype, qkv, qkv_row_stride, q_bias, k_bias, v_bias, cos_table,
+                       sin_table, k_pool, v_pool, block_tables, table_stride, num_blocks, cu_seqlens,
+                       start_pos, batch, total_rows, max_ctx, layer, num_layers, num_q_heads,
+                       num_kv_heads, head_dim, block_size, sm_scale, out, out_row_stride, true,
+                       workspace, workspace_bytes);
+}
+
 
 // ---- the model loop's small kernels (model_ops.hip) ----
 

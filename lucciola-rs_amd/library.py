@@ -51,6 +51,10 @@ SIGNATURES = {
     "luc_paged_prefill": (_i32, [_vp, _vp, _i32, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                  _vp, _i32, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32,
                                  _i32, _i32, _i32, _f32, _vp, _i64]),
+    "luc_paged_prefill_workspace_size": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32]),
+    "luc_paged_prefill_split": (_i32, [_vp, _vp, _i32, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                       _vp, _i32, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32,
+                                       _i32, _i32, _i32, _f32, _vp, _i64, _vp, _sz]),
     "luc_rmsnorm": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _f32, _i32, _i32]),
     "luc_silu_mul": (_i32, [_vp, _vp, _i32, _vp, _i32, _i32]),
     "luc_gemv": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32]),
@@ -118,7 +122,9 @@ def dtype_code(t: torch.Tensor) -> int:
 
 
 def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device address of a tensor for a c_void_p argument (argtypes convert the
+    int; a c_void_p object per argument would cost more than the launch)."""
+    return None if t is None else t.data_ptr()
 
 
 def pool_pages(pool, num_layers, num_kv_heads, head_dim) -> int:
@@ -132,7 +138,7 @@ def pool_pages(pool, num_layers, num_kv_heads, head_dim) -> int:
 def _stream(stream):
     if stream is None:
         stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return stream.cuda_stream
 
 
 class LucAttn:
@@ -247,16 +253,27 @@ class LucAttn:
                       cu_seqlens, start_pos, total_rows, max_ctx, layer, num_layers, hq, hkv,
                       head_dim, sm_scale, out, qkv_row_stride=None, out_row_stride=None,
                       block_size=16, stream=None, num_blocks=None):
-        """luc_paged_prefill: rope + cache write + causal attention of packed
-        prompts (cu_seqlens [B+1], start_pos [B] device int32)."""
+        """luc_paged_prefill_split: rope + cache write + causal attention of
+        packed prompts (cu_seqlens [B+1], start_pos [B] device int32), with the
+        partials of its K splits in a buffer allocated here, on the launch's
+        stream."""
         nb = num_blocks if num_blocks is not None else pool_pages(k_pool, num_layers, hkv, head_dim)
-        self._check(self.lib.luc_paged_prefill(
+        batch = start_pos.shape[0]
+        need = self.lib.luc_paged_prefill_workspace_size(batch, total_rows, max_ctx, hq, hkv, head_dim)
+        ws = None
+        if need:
+            if stream is None:
+                ws = torch.empty(need, dtype=torch.uint8, device=k_pool.device)
+            else:
+                with torch.cuda.stream(stream):
+                    ws = torch.empty(need, dtype=torch.uint8, device=k_pool.device)
+        self._check(self.lib.luc_paged_prefill_split(
             self.ctx, _stream(stream), dtype_code(k_pool), _p(qkv),
             qkv_row_stride if qkv_row_stride is not None else (hq + 2 * hkv) * head_dim,
             _p(q_bias), _p(k_bias), _p(v_bias), _p(cos), _p(sin), _p(k_pool), _p(v_pool),
-            _p(tables), tables.shape[-1], nb, _p(cu_seqlens), _p(start_pos), start_pos.shape[0],
+            _p(tables), tables.shape[-1], nb, _p(cu_seqlens), _p(start_pos), batch,
             total_rows, max_ctx, layer, num_layers, hq, hkv, head_dim, block_size, sm_scale,
-            _p(out), out_row_stride if out_row_stride is not None else hq * head_dim))
+            _p(out), out_row_stride if out_row_stride is not None else hq * head_dim, _p(ws), need))
 
     # ---- the model loop's small kernels ----
     def rmsnorm(self, out, x, weight, eps, stream=None):

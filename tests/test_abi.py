@@ -262,6 +262,27 @@ def test_prefill_argument_checks(cdll):
     assert call(batch=0) == 0 and call(total=0) == 0
 
 
+def test_prefill_split_workspace(cdll):
+    """Launches that fill the chip need no workspace; the others get one that
+    holds an f32 row and (max, sum) per split, row and head, are refused with a
+    smaller or misaligned one, and bad sizes ask for nothing."""
+    size = cdll.luc_paged_prefill_workspace_size
+    assert size(4, 8192, 2048, 14, 2, 64) == 0            # 448 workgroups
+    need = size(1, 512, 8512, 12, 2, 128)
+    per_split = 512 * 12 * (128 + 2) * 4
+    assert need % per_split == 0 and 2 <= need // per_split <= 64
+    assert size(1, 512, 8512, 12, 2, 80) == size(1, 0, 8512, 12, 2, 128) == size(1, 512, 8512, 18, 2, 64) == 0
+
+    def call(ws, n):
+        return cdll.luc_paged_prefill_split(
+            ctypes.c_void_p(1), None, 0, ctypes.c_void_p(256), 16 * 128, None, None, None,
+            ctypes.c_void_p(16), ctypes.c_void_p(16), ctypes.c_void_p(256), ctypes.c_void_p(512),
+            ctypes.c_void_p(16), 600, 600, ctypes.c_void_p(16), ctypes.c_void_p(16), 1, 512, 8512, 0, 1,
+            12, 2, 128, 16, 0.1, ctypes.c_void_p(256), 12 * 128, ws, n)
+    assert call(None, 0) == -5 and call(ctypes.c_void_p(256), need - 1) == -5
+    assert call(ctypes.c_void_p(128), need) == -1
+
+
 def test_sort_and_sample_argument_checks(cdll):
     """luc_sort_and_sample rejects on the host: top_k outside the built
     candidate sizes (the reference's "Unsupported candidate size"), bf16 only,

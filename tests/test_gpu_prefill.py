@@ -183,3 +183,33 @@ def test_prefill_long_prompt_beyond_max_ctx_all_flagged(orc, luc):
     assert np.array_equal(got["k_pool"], want["k_pool"]) and np.array_equal(got["v_pool"], want["v_pool"])
     err = float(np.max(np.abs(o[:30] - orc.to_f32(want["out"], "bf16")[:30])))
     assert err <= TOL["bf16"]
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (8, 8, 128), (16, 2, 128)])
+@pytest.mark.parametrize("rows,starts", [([1, 36, 37], [895, 128, 0]), ([2, 300], [767, 90]),
+                                         ([70], [1978])])
+def test_prefill_split_contexts(orc, luc, hq, hkv, d, rows, starts):
+    """Contexts cut into K splits: rows that end on, before and past a split
+    boundary, a sequence shorter than one split beside longer ones, and a tile
+    whose rows lie on both sides of a boundary; the unsplit entry point on the
+    same inputs agrees to f32 rounding of the sums plus one storage rounding."""
+    cfg = wl.PrefillConfig("split", len(rows), 0, hq, hkv, d, "bf16", 0, 0, 0.5)
+    h = wl.host_prefill_inputs(cfg, seed=sum(rows) + d, rows=rows, starts=starts)
+    total = int(h.cu_seqlens[-1])
+    need = luc.lib.luc_paged_prefill_workspace_size(len(rows), total, h.max_ctx, hq, hkv, d)
+    assert need > 0, "these sizes are meant to split"
+    got = gpu_prefill(luc, h)
+    assert_prefill_matches(orc, got, oracle_prefill(orc, luc, h), "bf16")
+    luc_size = luc.lib.luc_paged_prefill_workspace_size
+    try:
+        luc.lib.luc_paged_prefill_workspace_size = lambda *a: 0
+        split = luc.lib.luc_paged_prefill_split
+        luc.lib.luc_paged_prefill_split = lambda *a: luc.lib.luc_paged_prefill(*a[:-2])
+        whole = gpu_prefill(luc, h)
+    finally:
+        luc.lib.luc_paged_prefill_workspace_size, luc.lib.luc_paged_prefill_split = luc_size, split
+    for name in ("qkv", "k_pool", "v_pool"):
+        assert np.array_equal(got[name], whole[name])
+    a, b = orc.to_f32(got["out"], "bf16"), orc.to_f32(whole["out"], "bf16")
+    # p and the output round to bf16 (2^-9 each) around different maxima
+    assert np.max(np.abs(a - b)) <= 2 ** -7 * np.max(np.abs(b))
