@@ -369,11 +369,12 @@ __device__ void gemv_impl(uint16_t* y, const uint16_t* in, const uint16_t* w, co
 }  // namespace luc
 
 // Rows per wave R and 8-element chunks per lane C (rows of up to 512 C
-// elements): eight, four or one row of up to 1024 elements (the 896-wide
-// hidden state of the lm_head, gate/up, q/k/v and o products; fewer rows per
-// wave when there are fewer rows), or one row of up to 5120 (the down product's 4864) or 8192;
-// the gate/up pairs take four rows of up to 1024 or two of up to 5120 or 8192
-// (two outputs or one).
+// elements).  A lane's C chunk loads are unconditional, so chunks past a row's
+// end cost issue slots and L1 requests: C steps finely (1, 2, 3, 4, 6, 8, 10, 12,
+// 16), and R is what keeps about 16 chunks of weights in flight per lane while
+// there are waves to fill the chip with.  Gate/up at 8192 x 2 rows of 2048: 13.1
+// us on r4c4 (5.1 TB/s) against 41.9 with ten chunks a lane and two rows (r2c10,
+// 1.6 TB/s); q/k/v at 3072 rows of 2048: 5.1 us on r2c4 against 13.0 (r1c10).
 #define LUC_GEMV_KERNEL(NAME, PRE, POST, R, C)                                                    \
   extern "C" __global__ __launch_bounds__(luc::kGemvThreads) void NAME(uint16_t* y, const uint16_t* in, \
                                                          const uint16_t* w, const uint16_t* res,  \
@@ -381,21 +382,37 @@ __device__ void gemv_impl(uint16_t* y, const uint16_t* in, const uint16_t* w, co
                                                          int k) {                                 \
     luc::gemv_impl<R, C, PRE, POST>(y, in, w, res, nw, eps, n, k);                                \
   }
-LUC_GEMV_KERNEL(luc_gemv_bf16_r4c2, luc::kGemvPlain, luc::kGemvStore, 4, 2)
-LUC_GEMV_KERNEL(luc_gemv_bf16_r1c2, luc::kGemvPlain, luc::kGemvStore, 1, 2)
-LUC_GEMV_KERNEL(luc_gemv_bf16_r1c10, luc::kGemvPlain, luc::kGemvStore, 1, 10)
-LUC_GEMV_KERNEL(luc_gemv_bf16_r1c16, luc::kGemvPlain, luc::kGemvStore, 1, 16)
-LUC_GEMV_KERNEL(luc_rmsnorm_gemv_bf16_r4c2, luc::kGemvNorm, luc::kGemvStore, 4, 2)
-LUC_GEMV_KERNEL(luc_rmsnorm_gemv_bf16_r8c2, luc::kGemvNorm, luc::kGemvStore, 8, 2)
-LUC_GEMV_KERNEL(luc_rmsnorm_gemv_bf16_r1c2, luc::kGemvNorm, luc::kGemvStore, 1, 2)
-LUC_GEMV_KERNEL(luc_rmsnorm_gemv_bf16_r1c10, luc::kGemvNorm, luc::kGemvStore, 1, 10)
-LUC_GEMV_KERNEL(luc_rmsnorm_gemv_bf16_r1c16, luc::kGemvNorm, luc::kGemvStore, 1, 16)
-LUC_GEMV_KERNEL(luc_gate_up_silu_bf16_r4c2, luc::kGemvPlain, luc::kGemvSiluPair, 4, 2)
-LUC_GEMV_KERNEL(luc_gate_up_silu_bf16_r2c10, luc::kGemvPlain, luc::kGemvSiluPair, 2, 10)
-LUC_GEMV_KERNEL(luc_gate_up_silu_bf16_r2c16, luc::kGemvPlain, luc::kGemvSiluPair, 2, 16)
-LUC_GEMV_KERNEL(luc_rmsnorm_gate_up_silu_bf16_r4c2, luc::kGemvNorm, luc::kGemvSiluPair, 4, 2)
-LUC_GEMV_KERNEL(luc_rmsnorm_gate_up_silu_bf16_r2c10, luc::kGemvNorm, luc::kGemvSiluPair, 2, 10)
-LUC_GEMV_KERNEL(luc_rmsnorm_gate_up_silu_bf16_r2c16, luc::kGemvNorm, luc::kGemvSiluPair, 2, 16)
+#define LUC_GEMV_STORE(R, C)                                                                      \
+  LUC_GEMV_KERNEL(luc_gemv_bf16_r##R##c##C, luc::kGemvPlain, luc::kGemvStore, R, C)               \
+  LUC_GEMV_KERNEL(luc_rmsnorm_gemv_bf16_r##R##c##C, luc::kGemvNorm, luc::kGemvStore, R, C)
+#define LUC_GEMV_PAIR(R, C)                                                                       \
+  LUC_GEMV_KERNEL(luc_gate_up_silu_bf16_r##R##c##C, luc::kGemvPlain, luc::kGemvSiluPair, R, C)    \
+  LUC_GEMV_KERNEL(luc_rmsnorm_gate_up_silu_bf16_r##R##c##C, luc::kGemvNorm, luc::kGemvSiluPair, R, C)
+// (the same list in luc_attn.cpp, kGemvStoreShapes and kGemvPairShapes)
+LUC_GEMV_STORE(4, 2)
+LUC_GEMV_STORE(8, 2)
+LUC_GEMV_STORE(2, 1)
+LUC_GEMV_STORE(2, 2)
+LUC_GEMV_STORE(2, 3)
+LUC_GEMV_STORE(4, 3)
+LUC_GEMV_STORE(2, 4)
+LUC_GEMV_STORE(1, 6)
+LUC_GEMV_STORE(2, 6)
+LUC_GEMV_STORE(1, 8)
+LUC_GEMV_STORE(1, 10)
+LUC_GEMV_STORE(1, 12)
+LUC_GEMV_STORE(2, 16)
+LUC_GEMV_STORE(1, 16)
+LUC_GEMV_PAIR(4, 1)
+LUC_GEMV_PAIR(4, 2)
+LUC_GEMV_PAIR(4, 3)
+LUC_GEMV_PAIR(4, 4)
+LUC_GEMV_PAIR(2, 4)
+LUC_GEMV_PAIR(2, 6)
+LUC_GEMV_PAIR(2, 8)
+LUC_GEMV_PAIR(2, 10)
+LUC_GEMV_PAIR(2, 12)
+LUC_GEMV_PAIR(2, 16)
 
 extern "C" __global__ __launch_bounds__(256) void luc_rmsnorm_bf16(uint16_t* out, const uint16_t* in,
                                                                    const uint16_t* weight, float eps,

@@ -473,6 +473,17 @@ size_t prefill_workspace_bytes(const PrefillPlan& p, int total_rows, int hq, int
   return prefill_ml_bytes(p, total_rows, hq) + (size_t)p.splits * total_rows * hq * head_dim * 4;
 }
 
+// The built variants of the one-row products: rows per wave, 8-element chunks
+// per lane (model_ops.hip).
+struct GemvShape {
+  int rows, chunks;
+};
+constexpr GemvShape kGemvStoreShapes[] = {{4, 2}, {8, 2}, {2, 1}, {2, 2}, {2, 3}, {4, 3}, {2, 4}, {1, 6}, {2, 6}, {1, 8}, {1, 10}, {1, 12}, {2, 16}, {1, 16}};
+constexpr GemvShape kGemvPairShapes[] = {{4, 1}, {4, 2}, {4, 3}, {4, 4}, {2, 4}, {2, 6}, {2, 8}, {2, 10}, {2, 12}, {2, 16}};
+std::string gemv_variant(const GemvShape& v) {
+  return "_bf16_r" + std::to_string(v.rows) + "c" + std::to_string(v.chunks);
+}
+
 int launch_decode(DecodeLaunch& L, void* stream) {
   void* args[] = {&L.a};
   return launch(L.fn, L.grid, dim3(L.waves * 64), stream, args);
@@ -524,12 +535,10 @@ int luc_init(int device, const char* code_object_dir, luc_ctx** out_ctx) {
                                     "luc_argmax_bf16", "luc_gather_floor_d64",
                                     "luc_gather_floor_d128", "luc_stream_read"};
   for (int npl : {1, 2, 4, 8, 16}) names.push_back("luc_topk_filter_bf16_n" + std::to_string(npl));
-  for (const char* kind : {"luc_gemv", "luc_rmsnorm_gemv"})
-    for (const char* v : {"_bf16_r4c2", "_bf16_r1c2", "_bf16_r1c10", "_bf16_r1c16"})
-      names.push_back(std::string(kind) + v);
-  names.push_back("luc_rmsnorm_gemv_bf16_r8c2");
-  for (const char* kind : {"luc_gate_up_silu", "luc_rmsnorm_gate_up_silu"})
-    for (const char* v : {"_bf16_r4c2", "_bf16_r2c10", "_bf16_r2c16"}) names.push_back(std::string(kind) + v);
+  for (const GemvShape& v : kGemvStoreShapes)
+    for (const char* kind : {"luc_gemv", "luc_rmsnorm_gemv"}) names.push_back(kind + gemv_variant(v));
+  for (const GemvShape& v : kGemvPairShapes)
+    for (const char* kind : {"luc_gate_up_silu", "luc_rmsnorm_gate_up_silu"}) names.push_back(kind + gemv_variant(v));
   for (int k = 32; k <= 1024; k *= 2) names.push_back("luc_top_p_sample_" + std::to_string(k));
   for (const char* dt : {"bf16", "f16"}) {
     names.push_back(std::string("luc_rope_append_") + dt);
@@ -899,14 +908,40 @@ int luc_rmsnorm(luc_ctx* ctx, void* stream, int dtype, void* out, const void* in
 namespace {
 // The one-row products: `kind` names the kernel family, all with the
 // arguments (y, in, w, res, norm weight, eps, outputs, k).  Variant by shape:
-// rows of k <= 1024 on four rows per wave when there are at least 4096 of them,
-// eight with the norm when there are at least 65536 (the final norm + lm_head:
-// 47.0 against 48.0 us at 151936 x 896), else on one row per wave (q/k/v, o:
-// four times the waves to fill the chip with); rows of k <= 5120 or <= 8192 on one row per wave (ten or
-// sixteen 8-element chunks per lane).  The gate/up silu pairs (`pair`) take
-// two rows per output: four rows per wave for k <= 1024, else two (ten or
-// sixteen chunks per lane).  4 waves
-// per workgroup, one row group per wave.
+// the smallest chunk count built that covers k, and rows per wave by measured
+// time (us, weights from HBM; n x k):
+//   k <= 1024: two rows a wave (1152 x 896 with the norm: 2.9, one row 3.7),
+//     four from 4096 rows on, with the norm eight from 65536 (the final norm +
+//     lm_head, 151936 x 896: 46.1 on eight, 46.0 on four, 49.6 on two);
+//   k <= 2048: two (3072 x 2048: 5.1, one row 5.7; 2048 x 2048 without the norm:
+//     3.65 and 3.74; 151936 x 1536: 77 on two or four, one 113);
+//   k <= 3072: one (3072 x 3072: 5.2, two 5.6) or, from 4096 rows on, two
+//     (5120 x 3072 with the norm: 9.2, one 10.4);
+//   longer rows: one (896 x 4864: 4.05, two 4.85; 4608 x 3584: 12.7, two 13.7),
+//     above 6144 two from 1536 rows on (2048 x 8192: 8.8, one 9.4; 896 rows leave two-row waves too few).
+// The gate/up silu pairs (`pair`) take two rows per output: four rows up to
+// k = 2048 (8192 outputs: 13.1, two 13.45; 4864 x 896: 5.8 and 6.1) unless there are fewer
+// than 2048 outputs of more than 1536 (512 x 2048: two rows 3.6, four 4.35), else
+// two (8192 x 3072: 20.8, four 23.8).  4 waves per workgroup, one row group per
+// wave.
+GemvShape gemv_shape(bool pair, bool norm, int n, int k) {
+  const int need = (int)ceil_div(k, 512);
+  if (pair) {
+    if (need <= 3) return {4, need};
+    if (need == 4) return {n >= 2048 ? 4 : 2, 4};
+    return {2, need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10 : need <= 12 ? 12 : 16};
+  }
+  if (need <= 2) {
+    if (norm && n >= 65536) return {8, 2};
+    if (n >= 4096) return {4, 2};
+    return {2, need};
+  }
+  if (need <= 4) return {2, need};
+  if (need <= 6) return {n >= 4096 ? 2 : 1, 6};
+  if (need > 12) return {n >= 1536 ? 2 : 1, 16};
+  return {1, need <= 8 ? 8 : need <= 10 ? 10 : 12};
+}
+
 int gemv_launch(luc_ctx* ctx, void* stream, const char* kind, bool pair, void* y, const void* in,
                 const void* w, const void* residual, const void* norm_weight, float eps, int n, int k) {
   if (n < 0) return fail(LUC_E_INVALID, "%s: n %d < 0", kind, n);
@@ -918,19 +953,10 @@ int gemv_launch(luc_ctx* ctx, void* stream, const char* kind, bool pair, void* y
     return fail(LUC_E_INVALID, "%s: the input row, w and the norm weight must be 16-byte aligned", kind);
   if (n == 0) return LUC_OK;
   if (int rc = check_device(ctx)) return rc;
-  int outs_per_wave;
-  const char* variant;
-  if (pair) {
-    outs_per_wave = k <= 1024 ? 2 : 1;
-    variant = k <= 1024 ? "_bf16_r4c2" : k <= 5120 ? "_bf16_r2c10" : "_bf16_r2c16";
-  } else {
-    outs_per_wave = k <= 1024 && n >= 4096 ? 4 : 1;
-    if (norm_weight && k <= 1024 && n >= 65536) outs_per_wave = 8;
-    variant = k > 5120 ? "_bf16_r1c16" : k > 1024 ? "_bf16_r1c10" : outs_per_wave == 8 ? "_bf16_r8c2"
-              : outs_per_wave == 4 ? "_bf16_r4c2" : "_bf16_r1c2";
-  }
+  const GemvShape v = gemv_shape(pair, norm_weight != nullptr, n, k);
+  const int outs_per_wave = pair ? v.rows / 2 : v.rows;
   hipFunction_t fn;
-  if (int rc = get_fn(ctx, std::string(kind) + variant, &fn)) return rc;
+  if (int rc = get_fn(ctx, kind + gemv_variant(v), &fn)) return rc;
   const int64_t wgs = ceil_div(n, 4 * outs_per_wave);
   void* args[] = {&y, const_cast<void**>(&in), const_cast<void**>(&w), const_cast<void**>(&residual),
                   const_cast<void**>(&norm_weight), &eps, &n, &k};

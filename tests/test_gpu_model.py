@@ -153,6 +153,19 @@ def test_gate_up_silu_equals_unfused(luc, inter, k, norm):
     assert np.array_equal(from_dev(act), from_dev(gu[:inter]))
 
 
+@pytest.mark.parametrize("n,k", [
+    (67, 512), (67, 520), (2047, 1024), (67, 1536), (67, 1544), (2049, 2048), (513, 2056),
+    (4099, 2560), (67, 3072), (67, 3080), (67, 4096), (67, 4104), (67, 5120), (67, 5128),
+    (67, 6144), (1537, 6152), (67, 6152)])
+def test_one_row_products_at_variant_edges(luc, n, k):
+    """Every chunk count and row count of the dispatch, at the edges of its k
+    range and with n not a multiple of the rows a workgroup takes: the plain
+    product against f64, the fused ones against the unfused, bit for bit."""
+    test_gemv_against_f64(luc, n, k, True)
+    test_rmsnorm_gemv_equals_unfused(luc, n, k, False)
+    test_gate_up_silu_equals_unfused(luc, n, k, True)
+
+
 def test_gemv_rejects_bad_shapes(luc):
     """k outside [8, 8192] or not a multiple of 8, and mismatched operands,
     are refused before any launch."""
