@@ -270,6 +270,29 @@ int luc_paged_prefill_split(luc_ctx* ctx, void* stream, int dtype, void* qkv,
 int luc_rmsnorm(luc_ctx* ctx, void* stream, int dtype, void* out, const void* in,
                 const void* weight, float eps, int rows, int cols);
 
+/* y = round(x W^T) for `rows` rows x of k elements and W row-major [n][k]
+ * (bf16), f32 accumulation on MFMA -- Qwen2Model::matmul_bf16
+ * (src/models.rs:252-295) at m > 1.  k a multiple of 64, n of 4; x and W
+ * 16-byte aligned, y 8-byte. */
+int luc_prompt_gemm(luc_ctx* ctx, void* stream, int dtype, void* y, const void* x, const void* w,
+                    int rows, int n, int k);
+
+/* A decoder layer after its attention, for the rows of a prompt
+ * (Qwen2Model::forward_layer, src/models.rs:551-691), bf16:
+ *   h += att o_w^T (f32 sum, one rounding); x = RMSNorm(h) * post_norm;
+ *   act = silu(gate) * up of gate_up_w [2 intermediate][hidden];
+ *   h += act down_w^T; and, unless next_norm is NULL, x = RMSNorm(h) *
+ * next_norm, the next layer's normed input.  h, att and x are [rows][hidden], x
+ * scratch otherwise; hidden a multiple of 64 up to 8192, intermediate a
+ * multiple of 64; every operand 16-byte aligned.  The workspace (f32 partials of the
+ * products split over k, act) holds luc_prompt_mlp_workspace_size bytes, 256-byte aligned,
+ * contents arbitrary, used until the call's launches end. */
+size_t luc_prompt_mlp_workspace_size(int rows, int hidden, int intermediate);
+int luc_prompt_mlp(luc_ctx* ctx, void* stream, int dtype, void* h, const void* att, const void* o_w,
+                   const void* post_norm, float eps, const void* gate_up_w, const void* down_w,
+                   const void* next_norm, void* x, int rows, int hidden, int intermediate,
+                   void* workspace, size_t workspace_bytes);
+
 /* y = x W^T (+ residual) for one row x of k elements and W row-major
  * [n][k] (bf16): y[i] = round(sum_j x[j] W[i][j] (+ residual[i])), f32
  * accumulation in a fixed order -- the m = 1 case of Qwen2Model::matmul_bf16

@@ -24,8 +24,8 @@ LIB = os.path.join(HERE, "lib")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 
-KERNELS = ["rope_append", "paged_decode", "paged_decode_w8", "paged_prefill", "model_ops", "sampling",
-           "probe_gather"]
+KERNELS = ["rope_append", "paged_decode", "paged_decode_w8", "paged_prefill", "model_ops", "prompt_gemm",
+           "sampling", "probe_gather"]
 # code objects built from another object's source with extra flags
 KERNEL_SOURCES = {"paged_decode_w8": ("paged_decode", ["-DLUC_DECODE_WIDE"])}
 

@@ -60,8 +60,8 @@ int fail(int code, const char* fmt, ...) {
 
 constexpr const char* kCodeObjects[] = {"rope_append.hsaco",   "paged_decode.hsaco",
                                          "paged_decode_w8.hsaco", "paged_prefill.hsaco",
-                                         "model_ops.hsaco",     "sampling.hsaco",
-                                         "probe_gather.hsaco"};
+                                         "model_ops.hsaco",     "prompt_gemm.hsaco",
+                                         "sampling.hsaco",      "probe_gather.hsaco"};
 
 // Kernel-side constants (kept in step with csrc/kernels/paged_decode.hip):
 // four waves per workgroup, which share one split; tiles of 64 tokens
@@ -533,7 +533,8 @@ int luc_init(int device, const char* code_object_dir, luc_ctx** out_ctx) {
   }
   std::vector<std::string> names = {"luc_rmsnorm_bf16", "luc_silu_mul_bf16", "luc_embedding_bf16",
                                     "luc_argmax_bf16", "luc_gather_floor_d64",
-                                    "luc_gather_floor_d128", "luc_stream_read"};
+                                    "luc_gather_floor_d128", "luc_stream_read", "luc_gemm_store_bf16",
+                                    "luc_gemm_part_bf16", "luc_gemm_silu_bf16", "luc_reduce_norm_bf16"};
   for (int npl : {1, 2, 4, 8, 16}) names.push_back("luc_topk_filter_bf16_n" + std::to_string(npl));
   for (const GemvShape& v : kGemvStoreShapes)
     for (const char* kind : {"luc_gemv", "luc_rmsnorm_gemv"}) names.push_back(kind + gemv_variant(v));
@@ -986,6 +987,96 @@ int luc_gate_up_silu(luc_ctx* ctx, void* stream, int dtype, void* act, const voi
   if (dtype != LUC_BF16) return fail(LUC_E_UNSUPPORTED, "gate_up_silu: bf16 only");
   return gemv_launch(ctx, stream, norm_weight ? "luc_rmsnorm_gate_up_silu" : "luc_gate_up_silu", true,
                      act, x, w, nullptr, norm_weight, eps, intermediate, k);
+}
+
+namespace {
+// luc::GemmArgs of prompt_gemm.hip: the same fields in the same order.
+struct GemmArgs {
+  const void* x;
+  const void* w;
+  void* y;
+  int32_t m, n, k, splits, m_tiles, n_tiles;
+};
+// K ranges of a split product: enough workgroups (64 x 64 tiles) for two per
+// CU, each of at least four 64-deep steps; the partials grow with the count, and
+// luc_reduce_norm reads them all.
+int gemm_splits(int rows, int n, int k) {
+  const int64_t tiles = ceil_div(rows, 64) * ceil_div(n, 64);
+  return (int)std::max<int64_t>(1, std::min({2 * kCUs / tiles, (int64_t)k / 64 / 4, (int64_t)16}));
+}
+int launch_gemm(luc_ctx* ctx, void* stream, const char* kind, void* y, const void* x, const void* w,
+                int rows, int n, int k, int splits) {
+  hipFunction_t fn;
+  if (int rc = get_fn(ctx, kind, &fn)) return rc;
+  GemmArgs a{x, w, y, rows, n, k, splits, (int)ceil_div(rows, 64), (int)ceil_div(n, 64)};
+  // 8 (one per XCD) x blocks of 8 W row blocks x row tiles x splits
+  const int64_t grid = 8 * ceil_div(a.n_tiles, 8) * a.m_tiles * splits;
+  if (grid > INT32_MAX) return fail(LUC_E_INVALID, "%s: rows x n too large", kind);
+  void* args[] = {&a};
+  return launch(fn, dim3((unsigned)grid), dim3(256), stream, args);
+}
+int64_t prompt_part_bytes(int rows, int hidden, int inter) {
+  const int64_t s = std::max(gemm_splits(rows, hidden, hidden), gemm_splits(rows, hidden, inter));
+  return align256(s * rows * hidden * 4);
+}
+}  // namespace
+
+int luc_prompt_gemm(luc_ctx* ctx, void* stream, int dtype, void* y, const void* x, const void* w,
+                    int rows, int n, int k) {
+  if (!ctx) return fail(LUC_E_INVALID, "null context");
+  if (dtype != LUC_BF16) return fail(LUC_E_UNSUPPORTED, "prompt_gemm: bf16 only");
+  if (rows < 0 || n < 0) return fail(LUC_E_INVALID, "prompt_gemm: rows %d / n %d", rows, n);
+  if (k < 64 || k % 64 || n % 4)
+    return fail(LUC_E_UNSUPPORTED, "prompt_gemm: k %d (a multiple of 64), n %d (of 4)", k, n);
+  if (!y || !x || !w) return fail(LUC_E_INVALID, "prompt_gemm: null operand");
+  if (!aligned(x, 16) || !aligned(w, 16) || !aligned(y, 8))
+    return fail(LUC_E_INVALID, "prompt_gemm: x and w must be 16-byte aligned, y 8-byte");
+  if (rows == 0 || n == 0) return LUC_OK;
+  if (int rc = check_device(ctx)) return rc;
+  return launch_gemm(ctx, stream, "luc_gemm_store_bf16", y, x, w, rows, n, k, 1);
+}
+
+size_t luc_prompt_mlp_workspace_size(int rows, int hidden, int intermediate) {
+  if (rows <= 0 || hidden <= 0 || intermediate <= 0) return 0;
+  return (size_t)(prompt_part_bytes(rows, hidden, intermediate) + (int64_t)rows * intermediate * 2);
+}
+
+int luc_prompt_mlp(luc_ctx* ctx, void* stream, int dtype, void* h, const void* att, const void* o_w,
+                   const void* post_norm, float eps, const void* gate_up_w, const void* down_w,
+                   const void* next_norm, void* x, int rows, int hidden, int intermediate,
+                   void* workspace, size_t workspace_bytes) {
+  if (!ctx) return fail(LUC_E_INVALID, "null context");
+  if (dtype != LUC_BF16) return fail(LUC_E_UNSUPPORTED, "prompt_mlp: bf16 only");
+  if (rows < 0) return fail(LUC_E_INVALID, "prompt_mlp: rows %d", rows);
+  if (hidden < 64 || hidden > 8192 || hidden % 64 || intermediate < 64 || intermediate % 64)
+    return fail(LUC_E_UNSUPPORTED, "prompt_mlp: hidden %d (a multiple of 64 up to 8192), intermediate %d (of 64)",
+                hidden, intermediate);
+  if (!h || !att || !o_w || !post_norm || !gate_up_w || !down_w || !x)
+    return fail(LUC_E_INVALID, "prompt_mlp: null operand");
+  for (const void* p : {(const void*)h, att, o_w, post_norm, gate_up_w, down_w, next_norm, (const void*)x})
+    if (!aligned(p, 16)) return fail(LUC_E_INVALID, "prompt_mlp: operands must be 16-byte aligned");
+  if (rows == 0) return LUC_OK;
+  const size_t need = luc_prompt_mlp_workspace_size(rows, hidden, intermediate);
+  if (!workspace || workspace_bytes < need)
+    return fail(LUC_E_WORKSPACE, "workspace %zu bytes, %zu needed", workspace_bytes, need);
+  if (!aligned(workspace, 256)) return fail(LUC_E_INVALID, "workspace must be 256-byte aligned");
+  if (int rc = check_device(ctx)) return rc;
+  hipFunction_t reduce;
+  if (int rc = get_fn(ctx, "luc_reduce_norm_bf16", &reduce)) return rc;
+  void* part = workspace;
+  void* act = static_cast<char*>(workspace) + prompt_part_bytes(rows, hidden, intermediate);
+  auto add_norm = [&](int splits, const void* weight) {
+    void* args[] = {&h, &part, &splits, &x, &weight, &eps, &rows, &hidden};
+    return launch(reduce, dim3(rows), dim3(256), stream, args);
+  };
+  const int so = gemm_splits(rows, hidden, hidden), sd = gemm_splits(rows, hidden, intermediate);
+  if (int rc = launch_gemm(ctx, stream, "luc_gemm_part_bf16", part, att, o_w, rows, hidden, hidden, so)) return rc;
+  if (int rc = add_norm(so, post_norm)) return rc;
+  if (int rc = launch_gemm(ctx, stream, "luc_gemm_silu_bf16", act, x, gate_up_w, rows, intermediate, hidden, 1))
+    return rc;
+  if (int rc = launch_gemm(ctx, stream, "luc_gemm_part_bf16", part, act, down_w, rows, hidden, intermediate, sd))
+    return rc;
+  return add_norm(sd, next_norm);
 }
 
 int luc_silu_mul(luc_ctx* ctx, void* stream, int dtype, void* gate_up, int rows, int intermediate) {

@@ -56,6 +56,10 @@ SIGNATURES = {
                                        _vp, _i32, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32,
                                        _i32, _i32, _i32, _f32, _vp, _i64, _vp, _sz]),
     "luc_rmsnorm": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _f32, _i32, _i32]),
+    "luc_prompt_gemm": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32]),
+    "luc_prompt_mlp_workspace_size": (_sz, [_i32, _i32, _i32]),
+    "luc_prompt_mlp": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _i32,
+                              _i32, _i32, _vp, _sz]),
     "luc_silu_mul": (_i32, [_vp, _vp, _i32, _vp, _i32, _i32]),
     "luc_gemv": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32]),
     "luc_rmsnorm_gemv": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _f32, _vp, _vp, _i32, _i32]),
@@ -291,6 +295,34 @@ class LucAttn:
             raise ValueError(f"{name}: w {tuple(w.shape)}, x {tuple(x.shape)}, y {tuple(y.shape)}: "
                              "want contiguous x [k], y [n] (and residual [n]) for w [n, k]")
         return n, k
+
+    def prompt_gemm(self, y, x, w, stream=None):
+        """luc_prompt_gemm: y = x w^T for the rows of x [rows, k] and w [n, k] bf16."""
+        rows, k = x.shape
+        n = w.shape[0]
+        if not (w.is_contiguous() and x.is_contiguous() and y.is_contiguous()) or \
+                w.shape[1] != k or tuple(y.shape) != (rows, n):
+            raise ValueError(f"prompt_gemm: w {tuple(w.shape)}, x {tuple(x.shape)}, y {tuple(y.shape)}")
+        self._check(self.lib.luc_prompt_gemm(self.ctx, _stream(stream), dtype_code(w), _p(y), _p(x),
+                                             _p(w), rows, n, k))
+
+    def prompt_mlp(self, h, att, o_w, post_norm, eps, gate_up_w, down_w, next_norm, x, workspace,
+                   stream=None):
+        """luc_prompt_mlp: a layer's rows h [rows, hidden] (in place) from its
+        attention output; x gets the next layer's normed input (next_norm None:
+        scratch).  workspace: uint8 of luc_prompt_mlp_workspace_size."""
+        rows, hidden = h.shape
+        inter = down_w.shape[1]
+        if not all(t.is_contiguous() for t in (h, att, o_w, gate_up_w, down_w, x)) or \
+                att.shape != h.shape or x.shape != h.shape or tuple(o_w.shape) != (hidden, hidden) or \
+                tuple(gate_up_w.shape) != (2 * inter, hidden) or down_w.shape[0] != hidden or \
+                post_norm.numel() != hidden or (next_norm is not None and next_norm.numel() != hidden):
+            raise ValueError(f"prompt_mlp: h {tuple(h.shape)}, att {tuple(att.shape)}, o_w {tuple(o_w.shape)}, "
+                             f"gate_up_w {tuple(gate_up_w.shape)}, down_w {tuple(down_w.shape)}")
+        self._check(self.lib.luc_prompt_mlp(
+            self.ctx, _stream(stream), dtype_code(h), _p(h), _p(att), _p(o_w), _p(post_norm), eps,
+            _p(gate_up_w), _p(down_w), _p(next_norm), _p(x), rows, hidden, inter, _p(workspace),
+            workspace.numel()))
 
     def gemv(self, y, x, w, residual=None, stream=None):
         """luc_gemv: y = x w^T (+ residual) for one row x [k] (or [1, k]) and

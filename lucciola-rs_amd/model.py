@@ -110,8 +110,10 @@ class Qwen2Model:
     """One sequence through the decoder: `forward(ids, cache_pos)` then
     `sample_greedy()`, or `generate` (models.rs:184-243).  The products of a
     single row (every decode step) are luc_gemv on the weights in the
-    reference's [out, in] layout ("*_w"); those of a prompt are hipBLASLt GEMMs
-    on a transposed copy ([in, out], contiguous: "*_t")."""
+    reference's [out, in] layout ("*_w"); those of a prompt are the MFMA products
+    of luc_prompt_gemm and luc_prompt_mlp on the same weights, or, for sizes that
+    these do not take (hidden or intermediate not a multiple of 64), hipBLASLt
+    GEMMs on a transposed copy ([in, out], contiguous: "*_t")."""
 
     def __init__(self, cfg: Qwen2Config, weights: dict, num_blocks: int | None = None,
                  max_positions: int | None = None, device="cuda", lib=None):
@@ -124,7 +126,8 @@ class Qwen2Model:
                              "(luc_gemv) take rows of at most that many elements")
         if cfg.hidden_size % cfg.num_attention_heads or d not in (64, 128):
             raise ValueError(f"unsupported head_dim {d}")
-        T = lambda bits: _dev(bits, self.device).t().contiguous()  # noqa: E731  [in, out]
+        H, I = cfg.hidden_size, cfg.intermediate_size
+        self.prompt_kernels = H % 64 == 0 and I % 64 == 0
         self.embed = _dev(weights["embed_tokens"], self.device)
         # [vocab, hidden] for the one-row logits: the embedding when tied
         self.lm_head_w = _dev(weights["lm_head"], self.device) if "lm_head" in weights else self.embed
@@ -134,15 +137,21 @@ class Qwen2Model:
             qb = _dev(lw["qkv_bias"], self.device)
             q_dim, k_dim = cfg.hidden_size, cfg.num_key_value_heads * d
             W = lambda name: _dev(lw[name], self.device)  # noqa: E731  [out, in]
-            self.layers.append({
+            L = {
                 "in_norm": _dev(lw["input_layernorm"], self.device),
-                "qkv_t": T(lw["qkv_proj"]), "qkv_w": W("qkv_proj"),
+                "qkv_w": W("qkv_proj"),
                 "q_bias": qb[:q_dim], "k_bias": qb[q_dim:q_dim + k_dim], "v_bias": qb[q_dim + k_dim:],
-                "o_t": T(lw["o_proj"]), "o_w": W("o_proj"),
+                "o_w": W("o_proj"),
                 "post_norm": _dev(lw["post_attention_layernorm"], self.device),
-                "gate_up_t": T(lw["gate_up_proj"]), "gate_up_w": W("gate_up_proj"),
-                "down_t": T(lw["down_proj"]), "down_w": W("down_proj"),
-            })
+                "gate_up_w": W("gate_up_proj"),
+                "down_w": W("down_proj"),
+            }
+            if not self.prompt_kernels:
+                for name in ("qkv", "o", "gate_up"):
+                    L[name + "_t"] = L[name + "_w"].t().contiguous()
+            if not self.prompt_kernels or I > GEMV_MAX_K:  # (one row: _layer)
+                L["down_t"] = L["down_w"].t().contiguous()
+            self.layers.append(L)
         max_pos = max_positions or cfg.max_position_embeddings
         self.max_positions = max_pos
         self.rope = RopeCache(max_pos, d, cfg.rope_theta, cfg.rope_scaling_factor, device=self.device,
@@ -224,6 +233,23 @@ class Qwen2Model:
         self.lib.silu_mul(gate_up, I)
         return h.addmm_(gate_up[:, :I], L["down_t"])
 
+    def _prompt_layers(self, h, attention):
+        """Every decoder layer on a prompt's rows h, in place."""
+        cfg = self.cfg
+        eps = cfg.rms_norm_eps
+        S, H = h.shape
+        x = torch.empty_like(h)
+        qkv = torch.empty(S, cfg.qkv_dim, dtype=h.dtype, device=h.device)
+        ws = torch.empty(self.lib.lib.luc_prompt_mlp_workspace_size(S, H, cfg.intermediate_size),
+                         dtype=torch.uint8, device=h.device)
+        self.lib.rmsnorm(x, h, self.layers[0]["in_norm"], eps)
+        for li, L in enumerate(self.layers):
+            self.lib.prompt_gemm(qkv, x, L["qkv_w"])
+            att = attention(li, qkv)
+            nxt = self.layers[li + 1]["in_norm"] if li + 1 < len(self.layers) else None
+            self.lib.prompt_mlp(h, att, L["o_w"], L["post_norm"], eps, L["gate_up_w"], L["down_w"],
+                                nxt, x, ws)
+
     # ---- forward (models.rs:693-830) ----
     def forward(self, input_ids, cache_pos: int) -> None:
         """Run the decoder over `input_ids` at positions cache_pos...; leaves the
@@ -238,7 +264,8 @@ class Qwen2Model:
         ids = torch.tensor([int(i) for i in input_ids], dtype=torch.int32, device=self.device)
         h = torch.empty(S, cfg.hidden_size, dtype=torch.bfloat16, device=self.device)
         self.lib.embedding(h, self.embed, ids)
-        for p in range(cache_pos, cache_pos + S):  # the pages of every position first
+        # the pages of every position first
+        for p in range(cache_pos - cache_pos % self.kv.block_size, cache_pos + S, self.kv.block_size):
             self.kv.prepare_for_step(p)
         if S == 1:
             self.pos.fill_(cache_pos)
@@ -248,6 +275,10 @@ class Qwen2Model:
             start = torch.tensor([cache_pos], dtype=torch.int32, device=self.device)
             attention = lambda li, qkv: self._attention_prefill(li, qkv, cache_pos, cu, start)  # noqa: E731
         n = cfg.num_hidden_layers
+        if S > 1 and self.prompt_kernels:
+            self._prompt_layers(h, attention)
+            self.hidden.copy_(h[S - 1:])
+            return
         for li in range(n - 1):
             h = self._layer(li, h, attention)
         if S == 1:  # the last down product writes self.hidden

@@ -587,3 +587,50 @@ def test_decode_graph_replays_the_eager_loop(qwen):
         assert tok == eager[s + 1], f"replay {s}: token {tok}, eager loop {eager[s + 1]}"
     assert int(gpu.pos.cpu().item()) == len(prompt) + 48
     say(f"  48 replays equal the eager loop's tokens (first {eager[1:6]})")
+
+
+@pytest.mark.parametrize("rows,hidden,inter", [
+    (2, 64, 64), (63, 128, 192), (64, 896, 4864), (65, 192, 512), (700, 896, 4864), (33, 2048, 320),
+    (130, 8192, 64)])
+def test_prompt_layer_products(luc, rows, hidden, inter):
+    """luc_prompt_gemm and luc_prompt_mlp at the edges of their tiles (64 rows,
+    64 columns), of the K splits and of the row length, against the same steps in
+    f64 with the roundings the kernels state (h, x, gate, up and act in bf16).
+    Every product's f32 sum rounds once, so an element may sit one bf16 unit off
+    where its exact value lies next to a rounding boundary, and each rounding
+    step passes such units on to what follows: 2^-7 of the row's scale bounds
+    the largest difference, and 1 / 64 of the elements may differ by more than a unit."""
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden + inter)
+
+    def mk(*shape, std=1.0, mean=0.0):
+        return (torch.randn(*shape, generator=gen, device="cuda") * std + mean).to(torch.bfloat16)
+
+    h, att = mk(rows, hidden), mk(rows, hidden)
+    o_w, gu_w = mk(hidden, hidden, std=hidden ** -0.5), mk(2 * inter, hidden, std=hidden ** -0.5)
+    down_w = mk(hidden, inter, std=inter ** -0.5)
+    n1, n2 = mk(hidden, std=0.1, mean=1.0), mk(hidden, std=0.1, mean=1.0)
+    eps = 1e-6
+    r = lambda t: t.to(torch.float32).to(torch.bfloat16).double()  # noqa: E731
+    norm = lambda t, w: r(t / torch.sqrt((t * t).mean(-1, keepdim=True) + eps) * w.double())  # noqa: E731
+    h1 = r(h.double() + att.double() @ o_w.double().t())
+    gu = r(norm(h1, n1) @ gu_w.double().t())
+    act = r(torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:])
+    h2 = r(h1 + act @ down_w.double().t())
+    want_x = norm(h2, n2)
+    x = torch.empty_like(h)
+    ws = torch.full((luc.lib.luc_prompt_mlp_workspace_size(rows, hidden, inter),), 255,
+                    dtype=torch.uint8, device="cuda")
+    say(f"  [gpu] prompt_mlp rows={rows} hidden={hidden} inter={inter}")
+    luc.prompt_mlp(h, att, o_w, n1, eps, gu_w, down_w, n2, x, ws)
+    n = (hidden // 2) // 4 * 4 + 4
+    y = torch.empty(rows, n, dtype=torch.bfloat16, device="cuda")
+    w = mk(n, hidden, std=hidden ** -0.5)
+    luc.prompt_gemm(y, att, w)
+    torch.cuda.synchronize()
+    for name, got, want in (("y", y, r(att.double() @ w.double().t())), ("h", h, h2), ("x", x, want_x)):
+        d = (got.double() - want).abs()
+        unit = torch.exp2(torch.floor(torch.log2(want.abs().clamp_min(1e-9))) - 7)
+        over = float((d > unit).double().mean())
+        say(f"  {name}: max {float(d.max()):.3e}, beyond a unit {over:.4f}")
+        assert float((d / want.abs().amax(-1, keepdim=True)).max()) <= 2 ** -7, name
+        assert over <= 1 / 64, name
