@@ -12,19 +12,26 @@
 // (matmul_bf16's beta = 1), and the RMSNorm of the new row for the product that
 // follows.
 //
-// A workgroup of 4 waves takes a tile of 64 rows of x and BN of W (64; 128 for the
-// gate/up pairs: 64 gates with their 64 ups), wave (wn, wm) the W rows BN/2 wn
-// .. and the x rows 32 wm ...  Both operands are K-contiguous, so a K step of 64 is
-// 128 bytes of every row, loaded straight into LDS (global_load_lds_dwordx4, one
-// wave-wide load = 8 rows) into a ring of 4 stages (3 for the pairs), up to three steps ahead; 16-byte chunk c
-// of tile row r sits at slot c ^ ((r >> 1) & 7), so a 16-lane pass of the operand
-// reads covers every LDS bank.  W is the MFMA's A operand and x its B
-// operand: a lane then holds 4 consecutive columns of one row of y.
+// A workgroup of 4 waves takes a tile of BM rows of x (64 or 128) and BN of W (64 or
+// 128; 128 for the gate/up pairs: 64 gates with their 64 ups), wave (wn, wm) the W
+// rows BN/2 wn .. and the x rows BM/2 wm ...  Both operands are K-contiguous, so a K
+// step of 64 is 128 bytes of every row, loaded straight into LDS
+// (global_load_lds_dwordx4, one wave-wide load = 8 rows) into a ring of as many stages
+// (2 to 4) as leave room for two workgroups per CU; 16-byte chunk c of tile row r sits
+// at slot c ^ ((r >> 1) & 7), so a 16-lane pass of the operand reads covers every LDS
+// bank.  W is the MFMA's A operand and x its B operand: a lane then holds 4
+// consecutive columns of one row of y.
 //
-// Qwen2.5-0.5B, 700 rows, per layer (us, kernel trace): q/k/v 7.9, o and down
-// 16.2 on average, gate/up with silu 29.2, the two reductions with their norms 4.7 each;
-// hipBLASLt with separate norm and silu kernels took 11.5, 11.5 + 28.5, 23.3 + 6.3 and
-// 3.9 each, with ten launches a layer queued from Python.
+// What bounds it: at these sizes a workgroup runs 14 to 76 steps, each a barrier, LDS reads and
+// loads from L2 (8 to 10 TB/s in all); larger tiles halve the reads and loads per
+// MFMA and win once the rows fill the chip with them (us, hidden 896, intermediate
+// 4864): gate/up 28.7 on 64-row tiles and 24.1 on 128 at 700 rows, 15.7 and 16.1 at
+// 200; down 49.0 and 33.8 at 2000 rows, 19.2 and 21.6 at 700.  Four stages at one workgroup per
+// CU are slower (gate/up 30.7).
+//
+// Qwen2.5-0.5B, 700 rows, per layer (us): q/k/v 8.8, o 7.3, gate/up with silu 24.1, down
+// 19.2, the two reductions with their norms 4.7 each; hipBLASLt with separate norm and
+// silu kernels took 11.5, 11.5, 23.3 + 6.3, 28.5 and 3.9 each, with ten launches a layer queued from Python.
 //
 // A prompt's rows are few (5 to some thousand), so the tiles are small to fill 256
 // CUs, and o and down, with N = hidden, are split over K as well.  The tiles of a W row
@@ -48,7 +55,7 @@ struct GemmArgs {
 };
 
 enum GemmEpi { kGemmStore = 0, kGemmPart = 1, kGemmSilu = 2 };
-constexpr int kGemmM = 64, kGemmK = 64;
+constexpr int kGemmK = 64;
 
 // The operand reads of two 16-k steps, not valid before the wait below.
 __device__ inline void gemm_read2(uint32_t a0, uint32_t a1, u32x4_t* x) {
@@ -63,13 +70,18 @@ __device__ inline void gemm_wait2(u32x4_t* x) {
   asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(x[0]), "+v"(x[1]) : "n"(N) : "memory");
 }
 
-template <int EPI>
+template <int N>
+struct GemmIC {  // a compile-time index passed to a generic lambda
+  static constexpr int value = N;
+};
+
+template <int EPI, int FN, int FM, int NS>
 __device__ void gemm_impl(const GemmArgs& A) {
-  constexpr int BN = EPI == kGemmSilu ? 128 : 64;
-  constexpr int FN = BN / 64;                       // 32-row W fragments per wave
-  constexpr int STAGE = (kGemmM + BN) * 2 * kGemmK;  // bytes
-  constexpr int LOADS = STAGE / 1024 / 4;           // wave-wide loads per wave and stage
-  constexpr int NS = EPI == kGemmSilu ? 3 : 4;      // stages: two workgroups per CU
+  constexpr int BN = 64 * FN, BM = 64 * FM;    // FN (FM) 32-row fragments of W (x) per wave
+  constexpr int CN = EPI == kGemmSilu ? 64 : BN;  // columns of y per workgroup
+  static_assert(EPI != kGemmSilu || FN == 2, "a wave's gates and their ups");
+  constexpr int STAGE = (BM + BN) * 2 * kGemmK;  // bytes
+  constexpr int LOADS = STAGE / 1024 / 4;        // wave-wide loads per wave and stage
   __shared__ __attribute__((aligned(16))) char s_ab[NS][STAGE];  // W rows, then x rows
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -81,7 +93,7 @@ __device__ void gemm_impl(const GemmArgs& A) {
   if (nt >= A.n_tiles) return;
   const int rem = q % per;
   const int mt = rem % A.m_tiles, split = rem / A.m_tiles;
-  const int n0 = nt * 64, m0 = mt * kGemmM;
+  const int n0 = nt * CN, m0 = mt * BM;
   const int steps_all = A.k / kGemmK;
   const int s0 = (int)((int64_t)steps_all * split / A.splits);
   const int steps = (int)((int64_t)steps_all * (split + 1) / A.splits) - s0;
@@ -116,13 +128,15 @@ __device__ void gemm_impl(const GemmArgs& A) {
   uint32_t rel[4];  // slot of 16-k step kk (fragments start at multiples of 32 rows: same key)
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) rel[kk] = lr * 128 + (((2 * kk + g) ^ ((lr >> 1) & 7)) << 4);
-  const uint32_t wrow = wn * (BN / 2) * 128, xrow = (BN + wm * 32) * 128;
+  const uint32_t wrow = wn * (BN / 2) * 128, xrow = (BN + wm * (BM / 2)) * 128;
 
-  f32x16 acc[FN];
+  f32x16 acc[FM][FN];
 #pragma unroll
-  for (int f = 0; f < FN; ++f)
+  for (int h = 0; h < FM; ++h)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[f][e] = 0.0f;
+    for (int f = 0; f < FN; ++f)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[h][f][e] = 0.0f;
 
 #pragma unroll
   for (int j = 0; j < NS - 1; ++j)
@@ -138,58 +152,69 @@ __device__ void gemm_impl(const GemmArgs& A) {
     __builtin_amdgcn_s_barrier();
     if (t + NS - 1 < steps) issue(t + NS - 1);
     const uint32_t base = (uint32_t)(uintptr_t)(const lds_char_g*)s_ab[t % NS];
-    u32x4_t a[FN][4], b[4];
+    u32x4_t a[FN][4], b[FM][4];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      gemm_read2(base + xrow + rel[2 * p], base + xrow + rel[2 * p + 1], b + 2 * p);
+#pragma unroll
+      for (int h = 0; h < FM; ++h)
+        gemm_read2(base + xrow + h * 4096 + rel[2 * p], base + xrow + h * 4096 + rel[2 * p + 1], b[h] + 2 * p);
 #pragma unroll
       for (int f = 0; f < FN; ++f)
         gemm_read2(base + wrow + f * 4096 + rel[2 * p], base + wrow + f * 4096 + rel[2 * p + 1], a[f] + 2 * p);
     }
-    gemm_wait2<2 + 2 * FN>(b);
+    auto half = [&](auto pc) __attribute__((always_inline)) {  // 16-k steps 2 p and 2 p + 1
+      constexpr int p = decltype(pc)::value;
+      constexpr int later = p == 0 ? 2 * (FN + FM) : 0;  // reads that may be outstanding
 #pragma unroll
-    for (int f = 0; f < FN; ++f) gemm_wait2<2 + 2 * FN>(a[f]);
+      for (int h = 0; h < FM; ++h) gemm_wait2<later>(b[h] + 2 * p);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+      for (int f = 0; f < FN; ++f) gemm_wait2<later>(a[f] + 2 * p);
 #pragma unroll
-      for (int f = 0; f < FN; ++f)
-        acc[f] = mfma32<kBF16>(__builtin_bit_cast(uint4, a[f][kk]), __builtin_bit_cast(uint4, b[kk]), acc[f]);
-    gemm_wait2<0>(b + 2);
+      for (int kk = 2 * p; kk < 2 * p + 2; ++kk)
 #pragma unroll
-    for (int f = 0; f < FN; ++f) gemm_wait2<0>(a[f] + 2);
+        for (int h = 0; h < FM; ++h)
 #pragma unroll
-    for (int kk = 2; kk < 4; ++kk)
-#pragma unroll
-      for (int f = 0; f < FN; ++f)
-        acc[f] = mfma32<kBF16>(__builtin_bit_cast(uint4, a[f][kk]), __builtin_bit_cast(uint4, b[kk]), acc[f]);
+          for (int f = 0; f < FN; ++f)
+            acc[h][f] = mfma32<kBF16>(__builtin_bit_cast(uint4, a[f][kk]), __builtin_bit_cast(uint4, b[h][kk]),
+                                      acc[h][f]);
+    };
+    half(GemmIC<0>{});
+    half(GemmIC<1>{});
   }
 
-  // lane: row m, columns nb + 8 i + 4 g .. + 3 (gate / up of the same in acc[0], acc[1])
-  const int m = m0 + wm * 32 + lr;
-  if (m >= A.m) return;
+  // lane: row m of fragment hh, columns nf + 8 i + 4 g .. + 3 of fragment f (silu:
+  // gate in f = 0, its up in f = 1)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int n = n0 + wn * 32 + 8 * i + 4 * g;
-    if (n >= A.n) continue;  // (n a multiple of 4)
-    if constexpr (EPI == kGemmPart) {
-      float* const y = (float*)A.y + ((int64_t)split * A.m + m) * A.n + n;
-      *(float4*)y = make_float4(acc[0][4 * i], acc[0][4 * i + 1], acc[0][4 * i + 2], acc[0][4 * i + 3]);
-    } else {
-      uint32_t o[4];
+  for (int hh = 0; hh < FM; ++hh) {
+    const int m = m0 + wm * (BM / 2) + hh * 32 + lr;
+    if (m >= A.m) break;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (EPI == kGemmSilu) {
-#pragma clang fp contract(off)
-          const float gt = St<kBF16>::load(St<kBF16>::store(acc[0][4 * i + j]));
-          const float up = St<kBF16>::load(St<kBF16>::store(acc[FN - 1][4 * i + j]));
-          const float s = gt / (1.0f + expf(-gt));
-          o[j] = St<kBF16>::store(s * up);
+    for (int f = 0; f < (EPI == kGemmSilu ? 1 : FN); ++f)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = n0 + wn * (CN / 2) + f * 32 + 8 * i + 4 * g;
+        if (n >= A.n) continue;  // (n a multiple of 4)
+        const f32x16& v = acc[hh][f];
+        if constexpr (EPI == kGemmPart) {
+          float* const y = (float*)A.y + ((int64_t)split * A.m + m) * A.n + n;
+          *(float4*)y = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
         } else {
-          o[j] = St<kBF16>::store(acc[0][4 * i + j]);
+          uint32_t o[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if constexpr (EPI == kGemmSilu) {
+#pragma clang fp contract(off)
+              const float gt = St<kBF16>::load(St<kBF16>::store(v[4 * i + j]));
+              const float up = St<kBF16>::load(St<kBF16>::store(acc[hh][FN - 1][4 * i + j]));
+              const float s = gt / (1.0f + expf(-gt));
+              o[j] = St<kBF16>::store(s * up);
+            } else {
+              o[j] = St<kBF16>::store(v[4 * i + j]);
+            }
+          }
+          *(uint2*)((uint16_t*)A.y + (int64_t)m * A.n + n) = make_uint2(o[0] | o[1] << 16, o[2] | o[3] << 16);
         }
       }
-      *(uint2*)((uint16_t*)A.y + (int64_t)m * A.n + n) = make_uint2(o[0] | o[1] << 16, o[2] | o[3] << 16);
-    }
   }
 }
 
@@ -260,15 +285,16 @@ __device__ void reduce_norm_impl(uint16_t* h, const float* part, int splits, uin
 
 }  // namespace luc
 
-extern "C" __global__ __launch_bounds__(256, 2) void luc_gemm_store_bf16(luc::GemmArgs a) {
-  luc::gemm_impl<luc::kGemmStore>(a);
-}
-extern "C" __global__ __launch_bounds__(256, 2) void luc_gemm_part_bf16(luc::GemmArgs a) {
-  luc::gemm_impl<luc::kGemmPart>(a);
-}
-extern "C" __global__ __launch_bounds__(256, 2) void luc_gemm_silu_bf16(luc::GemmArgs a) {
-  luc::gemm_impl<luc::kGemmSilu>(a);
-}
+#define LUC_GEMM(NAME, EPI, FN, FM, NS)                                          \
+  extern "C" __global__ __launch_bounds__(256, 2) void NAME(luc::GemmArgs a) {   \
+    luc::gemm_impl<luc::EPI, FN, FM, NS>(a);                                     \
+  }
+LUC_GEMM(luc_gemm_store_bf16, kGemmStore, 1, 1, 4)
+LUC_GEMM(luc_gemm_part_bf16, kGemmPart, 1, 1, 4)
+LUC_GEMM(luc_gemm_part_bf16_m128, kGemmPart, 2, 2, 2)
+LUC_GEMM(luc_gemm_silu_bf16, kGemmSilu, 2, 1, 3)
+LUC_GEMM(luc_gemm_silu_bf16_m128, kGemmSilu, 2, 2, 2)
+
 extern "C" __global__ __launch_bounds__(256) void luc_reduce_norm_bf16(uint16_t* h, const float* part,
                                                                        int splits, uint16_t* out,
                                                                        const uint16_t* weight, float eps,

@@ -534,7 +534,8 @@ int luc_init(int device, const char* code_object_dir, luc_ctx** out_ctx) {
   std::vector<std::string> names = {"luc_rmsnorm_bf16", "luc_silu_mul_bf16", "luc_embedding_bf16",
                                     "luc_argmax_bf16", "luc_gather_floor_d64",
                                     "luc_gather_floor_d128", "luc_stream_read", "luc_gemm_store_bf16",
-                                    "luc_gemm_part_bf16", "luc_gemm_silu_bf16", "luc_reduce_norm_bf16"};
+                                    "luc_gemm_part_bf16", "luc_gemm_part_bf16_m128", "luc_gemm_silu_bf16",
+                                    "luc_gemm_silu_bf16_m128", "luc_reduce_norm_bf16"};
   for (int npl : {1, 2, 4, 8, 16}) names.push_back("luc_topk_filter_bf16_n" + std::to_string(npl));
   for (const GemvShape& v : kGemvStoreShapes)
     for (const char* kind : {"luc_gemv", "luc_rmsnorm_gemv"}) names.push_back(kind + gemv_variant(v));
@@ -997,21 +998,33 @@ struct GemmArgs {
   void* y;
   int32_t m, n, k, splits, m_tiles, n_tiles;
 };
-// K ranges of a split product: enough workgroups (64 x 64 tiles) for two per
-// CU, each of at least four 64-deep steps; the partials grow with the count, and
-// luc_reduce_norm reads them all.
+// Tiles of 128 rows where the rows fill the chip with them (prompt_gemm.hip,
+// measured there): the gate/up pairs (38 row blocks of W and more) from 257 rows on, o and
+// down (128 x 128 tiles, a seventh of the workgroups) from 1024.
+int gemm_tile_rows(bool silu, int rows) { return rows >= (silu ? 257 : 1024) ? 128 : 64; }
+// K ranges of a split product: as many as keep an XCD's workgroups (its share of
+// the W row blocks, 8 apart, x row tiles x ranges) in one round of two per CU, each of at
+// least four 64-deep steps.  One more than a round costs another: down at 700 rows
+// takes 19.2 us in 2 ranges (44 workgroups per XCD), 22.7 in 3 (66).
 int gemm_splits(int rows, int n, int k) {
-  const int64_t tiles = ceil_div(rows, 64) * ceil_div(n, 64);
-  return (int)std::max<int64_t>(1, std::min({2 * kCUs / tiles, (int64_t)k / 64 / 4, (int64_t)16}));
+  const int tile = gemm_tile_rows(false, rows);
+  const int64_t per_xcd = ceil_div(ceil_div(n, tile), 8) * ceil_div(rows, tile);
+  return (int)std::max<int64_t>(1, std::min({2 * kCUs / 8 / per_xcd, (int64_t)k / 64 / 4, (int64_t)16}));
 }
-int launch_gemm(luc_ctx* ctx, void* stream, const char* kind, void* y, const void* x, const void* w,
+enum GemmKind { kGemmStore, kGemmPart, kGemmSilu };
+int launch_gemm(luc_ctx* ctx, void* stream, GemmKind kind, void* y, const void* x, const void* w,
                 int rows, int n, int k, int splits) {
+  const int tile = kind == kGemmStore ? 64 : gemm_tile_rows(kind == kGemmSilu, rows);
+  const char* name = kind == kGemmStore ? "luc_gemm_store_bf16"
+                     : kind == kGemmPart ? (tile == 64 ? "luc_gemm_part_bf16" : "luc_gemm_part_bf16_m128")
+                                         : (tile == 64 ? "luc_gemm_silu_bf16" : "luc_gemm_silu_bf16_m128");
   hipFunction_t fn;
-  if (int rc = get_fn(ctx, kind, &fn)) return rc;
-  GemmArgs a{x, w, y, rows, n, k, splits, (int)ceil_div(rows, 64), (int)ceil_div(n, 64)};
+  if (int rc = get_fn(ctx, name, &fn)) return rc;
+  const int cols = kind == kGemmPart ? tile : 64;  // of y per workgroup
+  GemmArgs a{x, w, y, rows, n, k, splits, (int)ceil_div(rows, tile), (int)ceil_div(n, cols)};
   // 8 (one per XCD) x blocks of 8 W row blocks x row tiles x splits
   const int64_t grid = 8 * ceil_div(a.n_tiles, 8) * a.m_tiles * splits;
-  if (grid > INT32_MAX) return fail(LUC_E_INVALID, "%s: rows x n too large", kind);
+  if (grid > INT32_MAX) return fail(LUC_E_INVALID, "%s: rows x n too large", name);
   void* args[] = {&a};
   return launch(fn, dim3((unsigned)grid), dim3(256), stream, args);
 }
@@ -1033,7 +1046,7 @@ int luc_prompt_gemm(luc_ctx* ctx, void* stream, int dtype, void* y, const void* 
     return fail(LUC_E_INVALID, "prompt_gemm: x and w must be 16-byte aligned, y 8-byte");
   if (rows == 0 || n == 0) return LUC_OK;
   if (int rc = check_device(ctx)) return rc;
-  return launch_gemm(ctx, stream, "luc_gemm_store_bf16", y, x, w, rows, n, k, 1);
+  return launch_gemm(ctx, stream, kGemmStore, y, x, w, rows, n, k, 1);
 }
 
 size_t luc_prompt_mlp_workspace_size(int rows, int hidden, int intermediate) {
@@ -1070,11 +1083,11 @@ int luc_prompt_mlp(luc_ctx* ctx, void* stream, int dtype, void* h, const void* a
     return launch(reduce, dim3(rows), dim3(256), stream, args);
   };
   const int so = gemm_splits(rows, hidden, hidden), sd = gemm_splits(rows, hidden, intermediate);
-  if (int rc = launch_gemm(ctx, stream, "luc_gemm_part_bf16", part, att, o_w, rows, hidden, hidden, so)) return rc;
+  if (int rc = launch_gemm(ctx, stream, kGemmPart, part, att, o_w, rows, hidden, hidden, so)) return rc;
   if (int rc = add_norm(so, post_norm)) return rc;
-  if (int rc = launch_gemm(ctx, stream, "luc_gemm_silu_bf16", act, x, gate_up_w, rows, intermediate, hidden, 1))
+  if (int rc = launch_gemm(ctx, stream, kGemmSilu, act, x, gate_up_w, rows, intermediate, hidden, 1))
     return rc;
-  if (int rc = launch_gemm(ctx, stream, "luc_gemm_part_bf16", part, act, down_w, rows, hidden, intermediate, sd))
+  if (int rc = launch_gemm(ctx, stream, kGemmPart, part, act, down_w, rows, hidden, intermediate, sd))
     return rc;
   return add_norm(sd, next_norm);
 }

@@ -591,7 +591,8 @@ def test_decode_graph_replays_the_eager_loop(qwen):
 
 @pytest.mark.parametrize("rows,hidden,inter", [
     (2, 64, 64), (63, 128, 192), (64, 896, 4864), (65, 192, 512), (700, 896, 4864), (33, 2048, 320),
-    (130, 8192, 64)])
+    (130, 8192, 64), (256, 320, 192), (257, 320, 192), (1023, 192, 512), (1025, 192, 512),
+    (1100, 896, 1024)])
 def test_prompt_layer_products(luc, rows, hidden, inter):
     """luc_prompt_gemm and luc_prompt_mlp at the edges of their tiles (64 rows,
     64 columns), of the K splits and of the row length, against the same steps in
