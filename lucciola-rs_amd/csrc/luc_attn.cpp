@@ -411,12 +411,19 @@ struct PrefillArgs {
 // Prefill work split.  A workgroup takes a chunk of 256 (row, head of the
 // group) columns of one (sequence, kv head) and one K split.  With fewer
 // chunks than CUs, the contexts are cut into splits of `tokens` positions
-// (a multiple of 128) so that the grid fills the chip.  The lengths are on the device;
-// the plan takes `batch` sequences of equal rows that end at max_ctx, which
-// for one sequence is exact.  Cost in 64-token blocks: a workgroup takes its
-// blocks plus kPrefillUnit (prologue, epilogue, partials); the launch, its
+// (a multiple of 128) so that the grid fills the chip.  The lengths are on the
+// device; the plan takes `batch` sequences of equal rows that end at max_ctx,
+// which for one sequence is exact.  Cost in 64-token blocks: a workgroup takes
+// its blocks plus kPrefillUnit (prologue, epilogue, partials); the launch, its
 // longest workgroup or, with more than a round of them, the mean load of a CU
-// plus half a workgroup of tail.  Depends only on the arguments.
+// plus half a workgroup of tail; and a split launch pays kPrefillMerge and, for every
+// split, 3/4 of a block of partials written and merged.  Measured against fixed lengths (us per
+// call): 512 rows after 8000, 12 and 2 heads of 128: 56.3 at the plan's 896 tokens,
+// 73.7 at 768 (264 workgroups), 57.6 at 1024, 284 whole; 128 rows after 2000, 14 and 2 of
+// 64: 22.2 at 256, 24.3 at 128, 24.6 at 512, 50 whole; 2500 rows of the same: 41.8 at 1024,
+// 52.5 at 384, 59.5 whole; 700 rows of the same: 21.5 at 256, 22.7 at 128, 27.1 whole; 1000
+// rows, 12 and 2 of 128: 33.3 at 256, 39.1 at 128.
+// Depends only on the arguments.
 constexpr int kPrefillCols = 256;    // columns per workgroup: 8 waves x 32 (paged_prefill.hip)
 struct PrefillPlan {
   int chunks = 0;  // per (sequence, kv head), at most
@@ -425,7 +432,7 @@ struct PrefillPlan {
 };
 constexpr int kPrefillSlots = kCUs;  // resident workgroups: one per CU
 constexpr int kPrefillUnit = 4;      // blocks
-constexpr int kPrefillMerge = 4;     // blocks: q's RoPE in the append kernel, the merge launch
+constexpr int kPrefillMerge = 2;     // blocks: q's RoPE in the append kernel, the merge launch
 constexpr int kMaxPrefillSplits = 64;
 PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_ctx) {
   PrefillPlan p;
@@ -435,31 +442,41 @@ PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_
   const int64_t n = ceil_div(seq_rows * group, kPrefillCols);  // chunks of a mean sequence
   const int64_t groups = (int64_t)batch * hkv;
   if (n * groups >= kPrefillSlots || max_ctx > (1 << 28)) return p;
+  // the context of every chunk of a sequence, or of 32 of them at equal distances
+  constexpr int kSamples = 32;
+  const int m = (int)std::min<int64_t>(n, kSamples);
   const int64_t prefix = std::max<int64_t>(max_ctx - seq_rows, 0);
+  uint32_t ctx[kSamples];
+  int64_t blocks = 0;
+  for (int i = 0; i < m; ++i) {
+    const int64_t c = m == n ? i : (2 * i + 1) * n / (2 * m);
+    ctx[i] = (uint32_t)(prefix + std::min(seq_rows, ceil_div((c + 1) * kPrefillCols, group)));
+    blocks += (ctx[i] + 63) / 64;
+  }
+  blocks = blocks * n * groups / m;
   int64_t best = INT64_MAX;
-  int64_t last_tokens = 0;
-  for (int s = 1; s <= kMaxPrefillSplits; s += s < 16 ? 1 : 4) {
-    const int64_t tokens = ceil_div(ceil_div(max_ctx, s), 128) * 128;
-    if (tokens == last_tokens) continue;
-    last_tokens = tokens;
-    int64_t units = 0, blocks = 0;
-    for (int64_t c = 0; c < n; ++c) {
-      const int64_t ctx = prefix + std::min(seq_rows, ceil_div((c + 1) * kPrefillCols, group));
-      units += ceil_div(ctx, tokens);
-      blocks += ceil_div(ctx, 64);
-    }
-    units *= groups;
-    blocks *= groups;
-    const int64_t unit = std::min<int64_t>(tokens, max_ctx) / 64 + kPrefillUnit;
+  // whole contexts first, then shorter splits (ties keep the longer)
+  uint32_t tokens = (uint32_t)ceil_div(max_ctx, 128) * 128;
+  while (true) {
+    const int64_t splits = ceil_div(max_ctx, tokens);
+    if (splits > kMaxPrefillSplits) break;
+    int64_t units = 0;
+    for (int i = 0; i < m; ++i) units += (ctx[i] + tokens - 1) / tokens;
+    units = ceil_div(units * n * groups, m);
+    const int64_t unit = ceil_div(std::min<int64_t>(tokens, max_ctx), 64) + kPrefillUnit;
     // in 1 / kPrefillSlots of a block
     int64_t cost = unit * kPrefillSlots;
     if (units > kPrefillSlots) cost = std::max(cost, blocks + kPrefillUnit * units + unit * kPrefillSlots / 2);
-    if (s > 1) cost += kPrefillMerge * kPrefillSlots;
+    if (splits > 1) cost += (4 * kPrefillMerge + 3 * splits) * kPrefillSlots / 4;
     if (cost < best) {
       best = cost;
-      p.splits = (int)ceil_div(max_ctx, tokens);
-      p.tokens = p.splits > 1 ? (int)tokens : INT32_MAX;
+      p.splits = (int)splits;
+      p.tokens = splits > 1 ? (int)tokens : INT32_MAX;
     }
+    // 128 tokens less, or an eighth above 2048
+    const uint32_t step = tokens > 2048 ? (tokens / 8 + 127) / 128 * 128 : 128;
+    if (tokens <= step) break;
+    tokens -= step;
   }
   return p;
 }
