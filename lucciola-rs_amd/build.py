@@ -36,8 +36,7 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 # per code object: the prefill kernels keep their MFMA results in ordinary
-# VGPRs (the scores go straight to the VALU; the two-heads-per-wave kernels
-# hold their K and V operands in AGPRs, read by the MFMAs directly)
+# VGPRs (the scores go straight to the VALU)
 KERNEL_FLAGS = {"paged_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 

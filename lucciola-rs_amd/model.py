@@ -12,6 +12,8 @@ Per layer (Qwen2Model::forward_layer, models.rs:434-691):
   gu     = norm @ gate_up_proj^T                        GEMM
   gate   = silu(gate) * up                              luc_silu_mul
   h      = gate @ down_proj^T + h                       GEMM, beta = 1
+For a prompt whose sizes fit them, luc_prompt_gemm is the q/k/v product and
+luc_prompt_mlp everything from o to the next layer's norm.
 For one row (a decode step) the products are GEMVs with the norms and silu * up
 fused into them, five launches a layer with the same bits as the unfused ones:
 luc_rmsnorm_gemv (q/k/v), luc_decode_step, luc_gemv (o, + h),
