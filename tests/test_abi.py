@@ -283,6 +283,35 @@ def test_prefill_split_workspace(cdll):
     assert call(ctypes.c_void_p(128), need) == -1
 
 
+def test_prompt_product_argument_checks(cdll):
+    """luc_prompt_gemm and luc_prompt_mlp reject on the host: bf16 only, sizes
+    their tiles do not take, null or misaligned operands, a short workspace;
+    no rows is a no-op."""
+    p = ctypes.c_void_p
+
+    def gemm(**kw):
+        args = dict(ctx=p(1), stream=None, dtype=0, y=p(256), x=p(512), w=p(1024), rows=5, n=64, k=128)
+        args.update(kw)
+        return cdll.luc_prompt_gemm(*args.values())
+    assert gemm(dtype=1) == gemm(k=96) == gemm(k=0) == gemm(n=66) == -2
+    assert gemm(x=None) == gemm(w=p(1028)) == gemm(y=p(260)) == gemm(rows=-1) == gemm(ctx=None) == -1
+    assert gemm(rows=0) == gemm(n=0) == 0
+
+    need = cdll.luc_prompt_mlp_workspace_size(5, 128, 192)
+    assert need >= 5 * (128 * 4 + 192 * 2) and cdll.luc_prompt_mlp_workspace_size(0, 128, 192) == 0
+
+    def mlp(**kw):
+        args = dict(ctx=p(1), stream=None, dtype=0, h=p(256), att=p(512), o=p(1024), n1=p(256), eps=1e-6,
+                    gu=p(256), down=p(256), n2=None, x=p(256), rows=5, hidden=128, inter=192,
+                    ws=p(256), ws_bytes=need)
+        args.update(kw)
+        return cdll.luc_prompt_mlp(*args.values())
+    assert mlp(dtype=1) == mlp(hidden=96) == mlp(hidden=8256) == mlp(inter=200) == -2
+    assert mlp(h=None) == mlp(n1=None) == mlp(n2=p(8)) == mlp(ws=p(128)) == mlp(ctx=None) == -1
+    assert mlp(ws=None) == mlp(ws_bytes=need - 1) == -5
+    assert mlp(rows=0) == 0
+
+
 def test_sort_and_sample_argument_checks(cdll):
     """luc_sort_and_sample rejects on the host: top_k outside the built
     candidate sizes (the reference's "Unsupported candidate size"), bf16 only,
