@@ -266,8 +266,10 @@ class Qwen2Model:
         ids = torch.tensor([int(i) for i in input_ids], dtype=torch.int32, device=self.device)
         h = torch.empty(S, cfg.hidden_size, dtype=torch.bfloat16, device=self.device)
         self.lib.embedding(h, self.embed, ids)
-        # the pages of every position first
-        for p in range(cache_pos - cache_pos % self.kv.block_size, cache_pos + S, self.kv.block_size):
+        # the pages of every position first, and of those before it that no step
+        # has reserved (prepare_for_step appends one page a call, whatever the gap)
+        reserved = len(self.kv.block_table_cpu) * self.kv.block_size
+        for p in range(reserved, cache_pos + S, self.kv.block_size):
             self.kv.prepare_for_step(p)
         if S == 1:
             self.pos.fill_(cache_pos)

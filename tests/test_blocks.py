@@ -3,9 +3,13 @@ through the C ABI, on the CPU: the reference's single-sequence behaviour
 (KVCache free list and prepare_for_step, src/layers/kv_cache.rs:73-76,
 106-122), then a model-based check of many sequences against a plain Python
 statement of the allocation rules."""
+import dataclasses
+
 import numpy as np
 import pytest
+import torch
 
+from lucciola_rs_amd import model
 from lucciola_rs_amd.engine import BlockManager
 from lucciola_rs_amd.library import LucError
 
@@ -136,3 +140,52 @@ def test_random_operations_against_the_rules(seed):
         assert bm.num_free == len(m.free)
         held = [p for r in m.rows for p in r]
         assert len(set(held)) == len(held) and len(held) + len(m.free) == n  # no page twice
+
+
+class _NoLaunch:
+    """Stands in for the library object: the model's host work runs, every
+    launch is left out, and each attention call's block table is kept."""
+
+    def __init__(self):
+        self.tables = []
+        self.lib = self
+
+    def rope_table(self, max_pos, head_dim, base, scale):
+        return torch.zeros(max_pos, head_dim // 2), torch.zeros(max_pos, head_dim // 2)
+
+    def workspace_size(self, *a):
+        return 0
+
+    def luc_prompt_mlp_workspace_size(self, *a):
+        return 0
+
+    def decode_step(self, *a, **kw):
+        self.tables.append(a[8].clone())
+
+    def paged_prefill(self, *a, **kw):
+        self.tables.append(a[8].clone())
+
+    def __getattr__(self, name):
+        return lambda *a, **kw: None
+
+
+@pytest.mark.parametrize("calls", [
+    [(40, 32)], [(100, 160)], [(5, 0), (20, 40)], [(64, 700)], [(1, 700)], [(2, 33)],
+    [(33, 0), (1, 33), (1, 34)], [(16, 0), (16, 16), (1, 32), (40, 100)]])
+def test_model_reserves_the_pages_of_every_position(calls):
+    """Qwen2Model.forward at any start position, also past the reserved pages
+    (a prefix loaded straight into the pools): when the attention runs, the
+    table holds the pages 0, 1, 2, ... of every position up to the last row, none
+    twice and none missing."""
+    cfg = dataclasses.replace(model.QWEN25_05B, hidden_size=128, intermediate_size=128,
+                              num_attention_heads=2, num_key_value_heads=1, num_hidden_layers=1,
+                              vocab_size=64)
+    lib = _NoLaunch()
+    m = model.Qwen2Model(cfg, model.random_weights(cfg, 0), max_positions=1024, device="cpu", lib=lib)
+    last = 0
+    for rows, pos in calls:
+        m.forward([1] * rows, pos)
+        last = max(last, pos + rows)
+        pages = -(-last // 16)
+        assert m.kv.block_table_cpu == list(range(pages))
+        assert lib.tables[-1].reshape(-1)[:pages].tolist() == list(range(pages))
