@@ -382,27 +382,28 @@ __device__ void gemv_impl(uint16_t* y, const uint16_t* in, const uint16_t* w, co
                                                          int k) {                                 \
     luc::gemv_impl<R, C, PRE, POST>(y, in, w, res, nw, eps, n, k);                                \
   }
-#define LUC_GEMV_STORE(R, C)                                                                      \
-  LUC_GEMV_KERNEL(luc_gemv_bf16_r##R##c##C, luc::kGemvPlain, luc::kGemvStore, R, C)               \
+#define LUC_GEMV_PLAIN(R, C) \
+  LUC_GEMV_KERNEL(luc_gemv_bf16_r##R##c##C, luc::kGemvPlain, luc::kGemvStore, R, C)
+#define LUC_GEMV_NORM(R, C) \
   LUC_GEMV_KERNEL(luc_rmsnorm_gemv_bf16_r##R##c##C, luc::kGemvNorm, luc::kGemvStore, R, C)
+#define LUC_GEMV_STORE(R, C) LUC_GEMV_PLAIN(R, C) LUC_GEMV_NORM(R, C)
 #define LUC_GEMV_PAIR(R, C)                                                                       \
   LUC_GEMV_KERNEL(luc_gate_up_silu_bf16_r##R##c##C, luc::kGemvPlain, luc::kGemvSiluPair, R, C)    \
   LUC_GEMV_KERNEL(luc_rmsnorm_gate_up_silu_bf16_r##R##c##C, luc::kGemvNorm, luc::kGemvSiluPair, R, C)
-// (the same list in luc_attn.cpp, kGemvStoreShapes and kGemvPairShapes)
+// (the same lists in luc_attn.cpp, kGemvStoreShapes and kGemvPairShapes)
 LUC_GEMV_STORE(4, 2)
-LUC_GEMV_STORE(8, 2)
 LUC_GEMV_STORE(2, 1)
 LUC_GEMV_STORE(2, 2)
 LUC_GEMV_STORE(2, 3)
-LUC_GEMV_STORE(4, 3)
 LUC_GEMV_STORE(2, 4)
 LUC_GEMV_STORE(1, 6)
 LUC_GEMV_STORE(2, 6)
 LUC_GEMV_STORE(1, 8)
 LUC_GEMV_STORE(1, 10)
 LUC_GEMV_STORE(1, 12)
-LUC_GEMV_STORE(2, 16)
 LUC_GEMV_STORE(1, 16)
+LUC_GEMV_NORM(8, 2)
+LUC_GEMV_PLAIN(2, 16)  // (with the norm it spills: 27 VGPRs)
 LUC_GEMV_PAIR(4, 1)
 LUC_GEMV_PAIR(4, 2)
 LUC_GEMV_PAIR(4, 3)

@@ -495,7 +495,8 @@ size_t prefill_workspace_bytes(const PrefillPlan& p, int total_rows, int hq, int
 struct GemvShape {
   int rows, chunks;
 };
-constexpr GemvShape kGemvStoreShapes[] = {{4, 2}, {8, 2}, {2, 1}, {2, 2}, {2, 3}, {4, 3}, {2, 4}, {1, 6}, {2, 6}, {1, 8}, {1, 10}, {1, 12}, {2, 16}, {1, 16}};
+constexpr GemvShape kGemvStoreShapes[] = {{4, 2}, {2, 1}, {2, 2}, {2, 3}, {2, 4}, {1, 6}, {2, 6}, {1, 8}, {1, 10}, {1, 12}, {1, 16}};
+constexpr GemvShape kGemvNormOnly = {8, 2}, kGemvPlainOnly = {2, 16};
 constexpr GemvShape kGemvPairShapes[] = {{4, 1}, {4, 2}, {4, 3}, {4, 4}, {2, 4}, {2, 6}, {2, 8}, {2, 10}, {2, 12}, {2, 16}};
 std::string gemv_variant(const GemvShape& v) {
   return "_bf16_r" + std::to_string(v.rows) + "c" + std::to_string(v.chunks);
@@ -556,6 +557,8 @@ int luc_init(int device, const char* code_object_dir, luc_ctx** out_ctx) {
   for (int npl : {1, 2, 4, 8, 16}) names.push_back("luc_topk_filter_bf16_n" + std::to_string(npl));
   for (const GemvShape& v : kGemvStoreShapes)
     for (const char* kind : {"luc_gemv", "luc_rmsnorm_gemv"}) names.push_back(kind + gemv_variant(v));
+  names.push_back("luc_rmsnorm_gemv" + gemv_variant(kGemvNormOnly));
+  names.push_back("luc_gemv" + gemv_variant(kGemvPlainOnly));
   for (const GemvShape& v : kGemvPairShapes)
     for (const char* kind : {"luc_gate_up_silu", "luc_rmsnorm_gate_up_silu"}) names.push_back(kind + gemv_variant(v));
   for (int k = 32; k <= 1024; k *= 2) names.push_back("luc_top_p_sample_" + std::to_string(k));
@@ -937,7 +940,11 @@ namespace {
 //   k <= 3072: one (3072 x 3072: 5.2, two 5.6) or, from 4096 rows on, two
 //     (5120 x 3072 with the norm: 9.2, one 10.4);
 //   longer rows: one (896 x 4864: 4.05, two 4.85; 4608 x 3584: 12.7, two 13.7),
-//     above 6144 two from 1536 rows on (2048 x 8192: 8.8, one 9.4; 896 rows leave two-row waves too few).
+//     above 6144 without the norm two from 1536 rows on (2048 x 8192: 9.1, one 9.6;
+//     8192 x 6152: 26.3, one 28.8) except for 2049 .. 3072, which are three rounds of
+//     one-row waves and two, each twice as long, of two-row ones (2560 x 8192: one
+//     12.2, two 12.9); with the norm always one (3072 x 8192: 23.6, two 28.5, whose
+//     registers spill).
 // The gate/up silu pairs (`pair`) take two rows per output: four rows up to
 // k = 2048 (8192 outputs: 13.1, two 13.45; 4864 x 896: 5.8 and 6.1) unless there are fewer
 // than 2048 outputs of more than 1536 (512 x 2048: two rows 3.6, four 4.35), else
@@ -951,13 +958,14 @@ GemvShape gemv_shape(bool pair, bool norm, int n, int k) {
     return {2, need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10 : need <= 12 ? 12 : 16};
   }
   if (need <= 2) {
-    if (norm && n >= 65536) return {8, 2};
+    if (norm && n >= 65536) return kGemvNormOnly;
     if (n >= 4096) return {4, 2};
     return {2, need};
   }
   if (need <= 4) return {2, need};
   if (need <= 6) return {n >= 4096 ? 2 : 1, 6};
-  if (need > 12) return {n >= 1536 ? 2 : 1, 16};
+  if (need > 12)
+    return !norm && n >= 1536 && (n <= 2048 || n > 3072) ? kGemvPlainOnly : GemvShape{1, 16};
   return {1, need <= 8 ? 8 : need <= 10 ? 10 : 12};
 }
 

@@ -4,6 +4,7 @@ import ctypes
 import glob
 import os
 import re
+import subprocess
 
 import pytest
 import numpy as np
@@ -42,6 +43,32 @@ def test_code_objects_built_for_gfx950():
         data = open(path, "rb").read()
         assert data[:4] == b"\x7fELF"
         assert b"gfx950" in data
+
+
+def kernel_metadata(name):
+    """(kernel, spilled VGPRs, scratch bytes) of a built code object."""
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    notes = subprocess.run([os.path.join(rocm, "llvm", "bin", "llvm-readelf"), "--notes",
+                            os.path.join(library.lib_dir(), name + ".hsaco")],
+                           capture_output=True, text=True, check=True).stdout
+    out = []
+    for block in notes.split(".agpr_count:")[1:]:
+        field = lambda key: re.search(rf"^ *\.{key}: +(\S+)", block, re.M).group(1)  # noqa: E731
+        out.append((re.search(r"^    \.name: +(\S+)", block, re.M).group(1),
+                    int(field("vgpr_spill_count")), int(field("private_segment_fixed_size"))))
+    return out
+
+
+def test_kernels_that_wait_for_memory_do_not_spill():
+    """The one-row products that store rows, the prefill and the prompt
+    products keep every value in registers.  (The gate/up pairs of rows longer
+    than 6144 elements hold two rows of sixteen chunks and do not fit.)"""
+    for obj in ("model_ops", "paged_prefill", "prompt_gemm"):
+        kernels = kernel_metadata(obj)
+        assert len(kernels) >= 6
+        for kernel, spilled, scratch in kernels:
+            if not (kernel.endswith("r2c16") and "gate_up" in kernel):
+                assert (spilled, scratch) == (0, 0), kernel
 
 
 def test_abi_version_and_error_string():

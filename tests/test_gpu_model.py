@@ -156,7 +156,7 @@ def test_gate_up_silu_equals_unfused(luc, inter, k, norm):
 @pytest.mark.parametrize("n,k", [
     (67, 512), (67, 520), (2047, 1024), (67, 1536), (67, 1544), (2049, 2048), (513, 2056),
     (4099, 2560), (67, 3072), (67, 3080), (67, 4096), (67, 4104), (67, 5120), (67, 5128),
-    (67, 6144), (1537, 6152), (67, 6152)])
+    (67, 6144), (1537, 6152), (67, 6152), (2049, 6152), (3073, 6152)])
 def test_one_row_products_at_variant_edges(luc, n, k):
     """Every chunk count and row count of the dispatch, at the edges of its k
     range and with n not a multiple of the rows a workgroup takes: the plain
