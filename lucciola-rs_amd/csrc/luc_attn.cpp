@@ -442,6 +442,9 @@ PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_
   const int64_t n = ceil_div(seq_rows * group, kPrefillCols);  // chunks of a mean sequence
   const int64_t groups = (int64_t)batch * hkv;
   if (n * groups >= kPrefillSlots || max_ctx > (1 << 28)) return p;
+  // more rows than the sequences may hold: some sequence is flagged, and
+  // partials of all the rows would only take memory
+  if (total_rows > (int64_t)batch * max_ctx) return p;
   // the context of every chunk of a sequence, or of 32 of them at equal distances
   constexpr int kSamples = 32;
   const int m = (int)std::min<int64_t>(n, kSamples);

@@ -298,6 +298,9 @@ def test_prefill_split_workspace(cdll):
     need = size(1, 512, 8512, 12, 2, 128)
     per_split = 512 * 12 * (128 + 2) * 4
     assert need % per_split == 0 and 2 <= need // per_split <= 64
+    # more rows than max_ctx allows (a flagged sequence): no partials of all of them
+    assert size(1, 1000000, 1000, 14, 2, 64) == size(2, 2001, 1000, 14, 2, 64) == 0
+    assert 0 < size(1, 1000, 1000, 14, 2, 64) < 64 << 20
     assert size(1, 512, 8512, 12, 2, 80) == size(1, 0, 8512, 12, 2, 128) == size(1, 512, 8512, 18, 2, 64) == 0
 
     def call(ws, n):
