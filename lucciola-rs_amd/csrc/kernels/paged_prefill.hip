@@ -22,7 +22,7 @@
 // chunk c, sequence b, kv head h).  A split is a range of split_tokens
 // positions; the host cuts the contexts where the chunks alone leave CUs idle
 // (512 rows after 8000 cached, 12 q- and 2 kv-heads of 128: 24 chunks, 54 us a
-// call in 10 splits, 542 with every context in one workgroup of a head's rows).
+// call in 10 splits, 284 with every context whole).
 // Row i's position falls into the last split it reads: rows of positions below
 // split_tokens are finished by split 0, every other row's splits leave (max,
 // sum, unnormalised O) partials in the workspace for luc_prefill_merge.
@@ -87,7 +87,9 @@ struct PrefillArgs {
   float* ws_ml;  // [splits][total_rows][Hq] (max, sum), with splits > 1
   float* ws_o;   // [splits][total_rows][Hq][D]
   int32_t batch, layer, num_layers, hkv, max_ctx;
-  int32_t chunks;        // workgroups per (split, sequence, kv head)
+  int32_t chunks;        // workgroups per (split, sequence, kv head): gridDim.y ...
+  int32_t slots;         // ... or, if set, per (split, kv head), dealt by cu_seqlens
+  int32_t gblock;        // (sequence, kv head) pairs per block of them: gridDim.x
   int32_t num_blocks;    // pages per pool: table entries outside [0, num_blocks) are never used
   int32_t group;         // q-heads per kv head
   int32_t split_tokens;  // positions per split, a multiple of 128 (>= max_ctx: one split)
@@ -228,6 +230,7 @@ constexpr int kPrefillWaves = 8;
 template <int DT, int D>
 __device__ void prefill_impl(const PrefillArgs& A) {
   constexpr int W = kPrefillWaves;  // waves per workgroup: one 32-column tile each
+  constexpr int COLS = 32 * W;    // columns per chunk
   constexpr int BT = 64;          // tokens per block
   constexpr int CH = D / 8;       // 16-byte chunks per token row
   constexpr int ROWB = 2 * D;     // bytes per token row
@@ -255,16 +258,51 @@ __device__ void prefill_impl(const PrefillArgs& A) {
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // split-major, then the last (longest) chunk first; consecutive workgroups
-  // (which the hardware spreads over the XCDs) belong to different (b, h)
   const int G = A.group;
-  const int groups = A.batch * A.hkv;
-  int rem = blockIdx.x / groups;
-  const int bh = blockIdx.x - rem * groups;
-  const int split = rem / A.chunks;
-  const int chunk = A.chunks - 1 - (rem - split * A.chunks);
-  const int b = bh / A.hkv;
-  const int h = bh - b * A.hkv;
+  int b, h, split, chunk = 0, nchunks = 0;
+  if (A.slots) {
+    // grid (slot x kv head, 1, split): the chunks of sequence 0, then those of
+    // sequence 1, ..., and unused slots at the end (spread among the others they
+    // would leave some shader engines without work)
+    const int slot = blockIdx.x / A.hkv;
+    h = blockIdx.x - slot * A.hkv;
+    split = blockIdx.z;
+    b = -1;
+    for (int i0 = 0, before = 0; i0 < A.batch; i0 += 64) {
+      const int i = min(i0 + lane, A.batch - 1);
+      const int64_t cols = (int64_t)(A.cu_seqlens[i + 1] - A.cu_seqlens[i]) * G;
+      const int n = i0 + lane < A.batch && cols > 0 ? (int)((cols + COLS - 1) / COLS) : 0;
+      int upto = n;  // chunks of sequences i0 .. i
+#pragma unroll
+      for (int k = 1; k < 64; k <<= 1) {
+        const int x = __shfl_up(upto, k);
+        upto += lane >= k ? x : 0;
+      }
+      const uint64_t past = __builtin_amdgcn_ballot_w64(before + upto > slot);
+      if (past) {
+        const int l = __builtin_ctzll(past);
+        b = i0 + l;
+        nchunks = __builtin_amdgcn_readlane(n, l);
+        chunk = slot - before - (__builtin_amdgcn_readlane(upto, l) - nchunks);
+        break;
+      }
+      before += __builtin_amdgcn_readlane(upto, 63);
+    }
+    if (b < 0) return;
+  } else {
+    // grid (sequence and kv head within a block of them, chunk, split or block):
+    // the last (longest) chunk first; consecutive workgroups (which the hardware
+    // spreads over the XCDs) belong to different (b, h).  Several blocks are
+    // launched only without splits
+    const bool blocked = A.split_tokens == 0x7fffffff;
+    const int bh = blockIdx.x + (blocked ? blockIdx.z * A.gblock : 0);
+    split = blocked ? 0 : blockIdx.z;
+    nchunks = A.chunks;
+    chunk = nchunks - 1 - blockIdx.y;
+    b = bh / A.hkv;
+    h = bh - b * A.hkv;
+    if (b >= A.batch) return;
+  }
   const int row0 = A.cu_seqlens[b];
   const int nrows = A.cu_seqlens[b + 1] - row0;
   const int sp = A.start_pos[b];
@@ -315,7 +353,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
     // (such a sequence may have more columns than the grid has chunks: the
     // workgroups of its split 0 stride over all of them)
     if (split) return;
-    for (int64_t m = ((int64_t)chunk * W + w) * 32 + (lane & 31); m < ncols; m += (int64_t)A.chunks * W * 32) {
+    for (int64_t m = ((int64_t)chunk * W + w) * 32 + (lane & 31); m < ncols; m += (int64_t)nchunks * COLS) {
       const int r = (int)(m / G);
       const int qh = h * G + (int)(m - (int64_t)r * G);
       uint16_t* const orow = A.out + (int64_t)(row0 + r) * A.out_stride + (int64_t)qh * D;
@@ -335,10 +373,11 @@ __device__ void prefill_impl(const PrefillArgs& A) {
     }
     return;
   }
-  // within the bound: nrows <= max_ctx, and chunks covers its columns
-  if ((int64_t)chunk * (W * 32) >= ncols) return;
-  const int c0 = chunk * (W * 32);  // first column of the workgroup
-  const int last = sp + min((c0 + W * 32 - 1) / G, nrows - 1);  // last position of its rows
+  // within the bound: nrows <= max_ctx, and nchunks covers its columns
+  if (A.slots) chunk = nchunks - 1 - chunk;
+  if ((int64_t)chunk * COLS >= ncols) return;
+  const int c0 = chunk * COLS;  // first column of the workgroup
+  const int last = sp + min((c0 + COLS - 1) / G, nrows - 1);  // last position of its rows
   const int tok0 = split * A.split_tokens;
   if (tok0 > last) return;
   const int nkv = min(last + 1, tok0 + A.split_tokens);  // the split's tokens are tok0 .. nkv - 1

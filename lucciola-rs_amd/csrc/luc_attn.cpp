@@ -404,29 +404,40 @@ struct PrefillArgs {
   const float* sin_t;
   float* ws_ml;
   float* ws_o;
-  int32_t batch, layer, num_layers, hkv, max_ctx, chunks, num_blocks, group, split_tokens, total_rows;
+  int32_t batch, layer, num_layers, hkv, max_ctx, chunks, slots, gblock, num_blocks, group, split_tokens, total_rows;
   float qk_scale_log2;
 };
 
 // Prefill work split.  A workgroup takes a chunk of 256 (row, head of the
-// group) columns of one (sequence, kv head) and one K split.  With fewer
-// chunks than CUs, the contexts are cut into splits of `tokens` positions
-// (a multiple of 128) so that the grid fills the chip.  The lengths are on the
-// device; the plan takes `batch` sequences of equal rows that end at max_ctx,
-// which for one sequence is exact.  Cost in 64-token blocks: a workgroup takes
-// its blocks plus kPrefillUnit (prologue, epilogue, partials); the launch, its
-// longest workgroup or, with more than a round of them, the mean load of a CU
-// plus half a workgroup of tail; and a split launch pays kPrefillMerge and, for every
-// split, 3/4 of a block of partials written and merged.  Measured against fixed lengths (us per
-// call): 512 rows after 8000, 12 and 2 heads of 128: 56.3 at the plan's 896 tokens,
-// 73.7 at 768 (264 workgroups), 57.6 at 1024, 284 whole; 128 rows after 2000, 14 and 2 of
-// 64: 22.2 at 256, 24.3 at 128, 24.6 at 512, 50 whole; 2500 rows of the same: 41.8 at 1024,
-// 52.5 at 384, 59.5 whole; 700 rows of the same: 21.5 at 256, 22.7 at 128, 27.1 whole; 1000
-// rows, 12 and 2 of 128: 33.3 at 256, 39.1 at 128.
-// Depends only on the arguments.
+// group) columns of one (sequence, kv head) and one K split.  The lengths are on
+// the device: the plan takes `batch` sequences of equal rows that end at max_ctx,
+// which for one sequence is exact, and depends only on the arguments.
+//
+// K splits.  With fewer 256-column chunks than CUs, the contexts are cut into splits of
+// `tokens` positions (a multiple of 128) so that the grid fills the chip.  Cost in
+// 64-token blocks: a workgroup takes its blocks plus kPrefillUnit (prologue, epilogue,
+// partials); the launch, its longest workgroup or, with more than a round of them, the
+// mean load of a CU plus half a workgroup of tail; and a split launch pays
+// kPrefillMerge and, for every split, 3/4 of a block of partials written and merged.
+// Measured against fixed lengths (us per call): 512 rows after 8000, 12 and 2 heads of 128:
+// 56.3 at the plan's 896 tokens, 73.7 at 768 (264 workgroups), 57.6 at 1024, 284 whole;
+// 128 rows after 2000, 14 and 2 of 64: 22.8 at the plan's 384, 22.2 at
+// 256, 24.3 at 128, 24.6 at 512, 50 whole; 2500 rows of the same: 41.8 at
+// 1024, 52.5 at 384, 59.5 whole; 700 rows of the same: 21.5 at 256, 22.7 at 128, 27.1
+// whole; 1000 rows, 12 and 2 of 128: 33.3 at 256, 39.1 at 128.
+//
+// Grid.  Every (sequence, kv head) gets the chunks of the longest sequence the
+// arguments allow, min(total_rows, max_ctx) rows, or, where most of those would be idle
+// (more than 8 times the slots: 64 prompts of 128 rows after 4000, 64 and 8 heads of 128:
+// 1510 with the idle chunks, 1250 without), total_rows x group / columns + batch slots that the workgroups
+// deal among the sequences.  Short prompts of many sequences run in blocks of kPrefillBlock
+// (sequence, kv head) pairs, so that a pair's chunks run while its K and V are in L2 (64
+// prompts of 128 rows, 28 and 4 heads of 128: 81.3, in blocks 75.4).
 constexpr int kPrefillCols = 256;    // columns per workgroup: 8 waves x 32 (paged_prefill.hip)
 struct PrefillPlan {
   int chunks = 0;  // per (sequence, kv head), at most
+  int slots = 0;   // per kv head, instead
+  int gblock = 0;  // (sequence, kv head) pairs per block
   int splits = 1;
   int tokens = INT32_MAX;
 };
@@ -434,52 +445,67 @@ constexpr int kPrefillSlots = kCUs;  // resident workgroups: one per CU
 constexpr int kPrefillUnit = 4;      // blocks
 constexpr int kPrefillMerge = 2;     // blocks: q's RoPE in the append kernel, the merge launch
 constexpr int kMaxPrefillSplits = 64;
-PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_ctx) {
+constexpr int kPrefillBlock = 64;
+constexpr int kMaxGridYZ = 65535;
+constexpr int kMaxSlotSeqs = 512;  // (a workgroup reads the lengths of 64 sequences at a time)
+PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_ctx,
+                         bool may_split) {
   PrefillPlan p;
   const int64_t rows = std::min(total_rows, max_ctx);
-  p.chunks = (int)ceil_div(rows * group, kPrefillCols);
   const int64_t seq_rows = std::min<int64_t>(rows, ceil_div(total_rows, batch));
   const int64_t n = ceil_div(seq_rows * group, kPrefillCols);  // chunks of a mean sequence
   const int64_t groups = (int64_t)batch * hkv;
-  if (n * groups >= kPrefillSlots || max_ctx > (1 << 28)) return p;
-  // more rows than the sequences may hold: some sequence is flagged, and
-  // partials of all the rows would only take memory
-  if (total_rows > (int64_t)batch * max_ctx) return p;
-  // the context of every chunk of a sequence, or of 32 of them at equal distances
-  constexpr int kSamples = 32;
-  const int m = (int)std::min<int64_t>(n, kSamples);
-  const int64_t prefix = std::max<int64_t>(max_ctx - seq_rows, 0);
-  uint32_t ctx[kSamples];
-  int64_t blocks = 0;
-  for (int i = 0; i < m; ++i) {
-    const int64_t c = m == n ? i : (2 * i + 1) * n / (2 * m);
-    ctx[i] = (uint32_t)(prefix + std::min(seq_rows, ceil_div((c + 1) * kPrefillCols, group)));
-    blocks += (ctx[i] + 63) / 64;
-  }
-  blocks = blocks * n * groups / m;
-  int64_t best = INT64_MAX;
-  // whole contexts first, then shorter splits (ties keep the longer)
-  uint32_t tokens = (uint32_t)ceil_div(max_ctx, 128) * 128;
-  while (true) {
-    const int64_t splits = ceil_div(max_ctx, tokens);
-    if (splits > kMaxPrefillSplits) break;
-    int64_t units = 0;
-    for (int i = 0; i < m; ++i) units += (ctx[i] + tokens - 1) / tokens;
-    units = ceil_div(units * n * groups, m);
-    const int64_t unit = ceil_div(std::min<int64_t>(tokens, max_ctx), 64) + kPrefillUnit;
-    // in 1 / kPrefillSlots of a block
-    int64_t cost = unit * kPrefillSlots;
-    if (units > kPrefillSlots) cost = std::max(cost, blocks + kPrefillUnit * units + unit * kPrefillSlots / 2);
-    if (splits > 1) cost += (4 * kPrefillMerge + 3 * splits) * kPrefillSlots / 4;
-    if (cost < best) {
-      best = cost;
-      p.splits = (int)splits;
-      p.tokens = splits > 1 ? (int)tokens : INT32_MAX;
+  // (more rows than the sequences may hold: some sequence is flagged, and
+  // partials of all the rows would only take memory)
+  if (may_split && n * groups < kPrefillSlots && max_ctx <= (1 << 28) &&
+      total_rows <= (int64_t)batch * max_ctx) {
+    // the context of every chunk of a sequence, or of 32 of them at equal distances
+    constexpr int kSamples = 32;
+    const int m = (int)std::min<int64_t>(n, kSamples);
+    const int64_t prefix = std::max<int64_t>(max_ctx - seq_rows, 0);
+    uint32_t ctx[kSamples];
+    int64_t blocks = 0;
+    for (int i = 0; i < m; ++i) {
+      const int64_t c = m == n ? i : (2 * i + 1) * n / (2 * m);
+      ctx[i] = (uint32_t)(prefix + std::min(seq_rows, ceil_div((c + 1) * kPrefillCols, group)));
+      blocks += (ctx[i] + 63) / 64;
     }
-    // 128 tokens less, or an eighth above 2048
-    const uint32_t step = tokens > 2048 ? (tokens / 8 + 127) / 128 * 128 : 128;
-    if (tokens <= step) break;
-    tokens -= step;
+    blocks = blocks * n * groups / m;
+    int64_t best = INT64_MAX;
+    // whole contexts first, then shorter splits (ties keep the longer)
+    uint32_t tokens = (uint32_t)ceil_div(max_ctx, 128) * 128;
+    while (true) {
+      const int64_t splits = ceil_div(max_ctx, tokens);
+      if (splits > kMaxPrefillSplits) break;
+      int64_t units = 0;
+      for (int i = 0; i < m; ++i) units += (ctx[i] + tokens - 1) / tokens;
+      units = ceil_div(units * n * groups, m);
+      const int64_t unit = ceil_div(std::min<int64_t>(tokens, max_ctx), 64) + kPrefillUnit;
+      // in 1 / kPrefillSlots of a block
+      int64_t cost = unit * kPrefillSlots;
+      if (units > kPrefillSlots) cost = std::max(cost, blocks + kPrefillUnit * units + unit * kPrefillSlots / 2);
+      if (splits > 1) cost += (4 * kPrefillMerge + 3 * splits) * kPrefillSlots / 4;
+      if (cost < best) {
+        best = cost;
+        p.splits = (int)splits;
+        p.tokens = splits > 1 ? (int)tokens : INT32_MAX;
+      }
+      // 128 tokens less, or an eighth above 2048
+      const uint32_t step = tokens > 2048 ? (tokens / 8 + 127) / 128 * 128 : 128;
+      if (tokens <= step) break;
+      tokens -= step;
+    }
+  }
+  const int64_t chunks = ceil_div(rows * group, kPrefillCols);
+  const int64_t slots = (int64_t)total_rows * group / kPrefillCols + batch;
+  if ((batch <= kMaxSlotSeqs && batch * chunks > 8 * slots) || chunks > kMaxGridYZ ||
+      groups * chunks * (2 * kPrefillCols) > UINT32_MAX) {
+    p.slots = (int)std::min<int64_t>(slots, INT32_MAX);
+  } else {
+    p.chunks = (int)chunks;
+    const bool block = p.splits == 1 && groups >= kPrefillSlots && n * groups > kPrefillSlots && chunks <= 8 &&
+                       groups <= (int64_t)kPrefillBlock * kMaxGridYZ;
+    p.gblock = (int)(block ? kPrefillBlock : groups);
   }
   return p;
 }
@@ -813,11 +839,7 @@ static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64
     return fail(LUC_E_INVALID, "table_stride %d pages cannot hold max_ctx %d", table_stride, max_ctx);
   if (batch == 0 || total_rows == 0) return LUC_OK;
   const int group = num_q_heads / num_kv_heads;
-  PrefillPlan plan = prefill_plan(batch, num_kv_heads, group, total_rows, max_ctx);
-  if (!split) {
-    plan.splits = 1;
-    plan.tokens = INT32_MAX;
-  }
+  const PrefillPlan plan = prefill_plan(batch, num_kv_heads, group, total_rows, max_ctx, split);
   const size_t need = prefill_workspace_bytes(plan, total_rows, num_q_heads, head_dim);
   if (need && (!workspace || workspace_bytes < need))
     return fail(LUC_E_WORKSPACE, "workspace %zu bytes, %zu needed", workspace_bytes, need);
@@ -827,8 +849,13 @@ static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64
   hipFunction_t fn, merge;
   if (int rc = get_fn(ctx, "luc_prefill_" + suffix, &fn)) return rc;
   if (int rc = get_fn(ctx, "luc_prefill_merge_" + suffix, &merge)) return rc;
-  const int64_t grid = (int64_t)batch * num_kv_heads * plan.chunks * plan.splits;
-  if (grid > INT32_MAX) return fail(LUC_E_INVALID, "batch x kv heads x row tiles too large");
+  // slots: (slot and kv head, 1, split); else (pairs of a block, chunk, split or block)
+  const int64_t pairs = (int64_t)batch * num_kv_heads;
+  const int64_t grid_x = plan.slots ? (int64_t)plan.slots * num_kv_heads : plan.gblock;
+  const int64_t grid_z = plan.slots || plan.splits > 1 ? plan.splits : ceil_div(pairs, plan.gblock);
+  if (grid_x * 2 * kPrefillCols > UINT32_MAX || grid_z > kMaxGridYZ)
+    return fail(LUC_E_INVALID, "batch x kv heads x row tiles too large");
+  const dim3 grid((unsigned)grid_x, (unsigned)std::max(plan.chunks, 1), (unsigned)grid_z);
 
   // q's bias + RoPE runs in the attention kernel, which loads every row's q
   // anyway, when the bias and the rotation tables allow its 16-byte loads and
@@ -857,7 +884,7 @@ static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64
   p.start_pos = start_pos; p.out = out; p.out_stride = out_row_stride; p.batch = batch;
   p.q_bias = q_bias; p.cos_t = fuse_q ? cos_table : nullptr; p.sin_t = sin_table;
   p.layer = layer; p.num_layers = num_layers; p.hkv = num_kv_heads; p.max_ctx = max_ctx;
-  p.chunks = plan.chunks; p.num_blocks = num_blocks; p.group = group; p.split_tokens = plan.tokens;
+  p.chunks = plan.chunks; p.slots = plan.slots; p.gblock = plan.gblock; p.num_blocks = num_blocks; p.group = group; p.split_tokens = plan.tokens;
   p.total_rows = total_rows; p.qk_scale_log2 = sm_scale * 1.4426950408889634f;
   if (need) {
     p.ws_ml = static_cast<float*>(workspace);
@@ -865,7 +892,7 @@ static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64
                                       prefill_ml_bytes(plan, total_rows, num_q_heads));
   }
   void* args[] = {&p};
-  if (int rc = launch(fn, dim3((unsigned)grid), dim3(2 * kPrefillCols), stream, args)) return rc;
+  if (int rc = launch(fn, grid, dim3(2 * kPrefillCols), stream, args)) return rc;
   if (!need) return LUC_OK;
   // 3) the rows that several splits share (head_dim / 4 lanes per row and head)
   const int64_t items = (int64_t)total_rows * num_q_heads;
@@ -892,8 +919,8 @@ size_t luc_paged_prefill_workspace_size(int batch, int total_rows, int max_ctx, 
       num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > 8 || (head_dim != 64 && head_dim != 128))
     return 0;
   return prefill_workspace_bytes(
-      prefill_plan(batch, num_kv_heads, num_q_heads / num_kv_heads, total_rows, max_ctx), total_rows,
-      num_q_heads, head_dim);
+      prefill_plan(batch, num_kv_heads, num_q_heads / num_kv_heads, total_rows, max_ctx, true),
+      total_rows, num_q_heads, head_dim);
 }
 
 int luc_paged_prefill_split(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64_t qkv_row_stride,

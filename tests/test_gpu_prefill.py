@@ -213,3 +213,62 @@ def test_prefill_split_contexts(orc, luc, hq, hkv, d, rows, starts):
     a, b = orc.to_f32(got["out"], "bf16"), orc.to_f32(whole["out"], "bf16")
     # p and the output round to bf16 (2^-9 each) around different maxima
     assert np.max(np.abs(a - b)) <= 2 ** -7 * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("hq,hkv,d,batch,hi", [
+    (14, 2, 64, 20, 60), (8, 8, 128, 70, 40), (28, 4, 128, 65, 70), (64, 8, 64, 130, 40),
+    (12, 4, 64, 257, 30), (4, 4, 128, 600, 12)])
+def test_prefill_loose_bound_same_bits(orc, luc, hq, hkv, d, batch, hi):
+    """Ragged prompts (empty ones among them: the first, the last, two in a
+    row) under a bound max_ctx that is exact and one that is a hundred times too
+    large: the workgroups are dealt differently (all the chunks the bound
+    allows; slots dealt by cu_seqlens, at one and at several reads of 64 lengths;
+    blocks of 64 (sequence, kv head) pairs with a partial last one) and every
+    result is the same, bit for bit.  One sequence past the loose bound is
+    flagged, also where it alone has more rows than the others together."""
+    rng = np.random.default_rng(batch)
+    rows = rng.integers(1, hi, batch)
+    rows[[0, batch // 2, batch // 2 + 1, batch - 1]] = 0
+    cfg = wl.PrefillConfig("loose", batch, 0, hq, hkv, d, "bf16", 0, 0, 0.5)
+    h = wl.host_prefill_inputs(cfg, seed=batch, rows=rows, starts=rng.integers(0, 20, batch))
+    tight = gpu_prefill(luc, h)
+    wide = wl.replace(h, tables=np.pad(h.tables, ((0, 0), (0, 100 * hi // 16)),
+                                       constant_values=int(h.tables.max())))
+    loose = gpu_prefill(luc, wide, max_ctx=100 * hi)
+    for name in tight:
+        assert np.array_equal(tight[name], loose[name]), name
+    o = orc.to_f32(tight["out"], "bf16")
+    assert np.all(np.isfinite(o))
+    # the last sequence now longer than the bound
+    rows[-1] = 100 * hi + 7
+    h = wl.host_prefill_inputs(cfg, seed=batch, rows=rows, starts=np.zeros(batch, int), poison=False)
+    got = gpu_prefill(luc, h, max_ctx=100 * hi)
+    o = orc.to_f32(got["out"], "bf16")
+    n = int(h.cu_seqlens[-2])
+    assert np.all(np.isfinite(o[:n])) and np.all(np.isnan(o[n:]))
+
+
+def test_prefill_many_prompts_under_a_long_bound(orc, luc):
+    """1024 prompts of 32 rows, 64 and 8 heads, and a bound of all the rows in
+    one sequence: more than 2^32 threads, were every sequence given the chunks
+    that the bound allows.  The same bits as under the exact bound."""
+    cfg = wl.PrefillConfig("bound", 1024, 32, 64, 8, 64, "bf16", 0, 0, 0.5)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    qkv = torch.randn(1024 * 32, cfg.row, generator=gen, device="cuda").to(torch.bfloat16)
+    tables = torch.zeros(1024, 32768 // 16, dtype=torch.int32, device="cuda")
+    tables[:, :2] = torch.randperm(2048, generator=gen, device="cuda").to(torch.int32).view(1024, 2)
+    cu = torch.arange(1025, dtype=torch.int32, device="cuda") * 32
+    start = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    rope = rope_cache(luc, 64)
+    results = []
+    for max_ctx in (32, 32768):
+        x, out = qkv.clone(), torch.zeros(1024 * 32, 64 * 64, dtype=torch.bfloat16, device="cuda")
+        pools = [torch.zeros(2048, 1, 8, 16, 64, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+        say(f"  [gpu] paged_prefill 1024 x 32 rows, max_ctx={max_ctx}")
+        luc.paged_prefill(x, None, None, None, rope.cos, rope.sin, *pools, tables, cu, start,
+                          1024 * 32, max_ctx, 0, 1, 64, 8, 64, sm_scale(64), out)
+        torch.cuda.synchronize()
+        results.append([x, out, *pools])
+    assert torch.isfinite(results[0][1]).all() and results[0][1].any(-1).all()
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
