@@ -16,7 +16,7 @@
 //
 // Work decomposition: the (prompt row, q-head of the group) pairs of a sequence
 // and kv head h, row-major (m = row * G + head, G = Hq / Hkv), in tiles of 32:
-// one tile per wave, chunks of 8 consecutive tiles per workgroup, so the K and
+// one tile per wave, chunks of 8 (or 4) consecutive tiles per workgroup, so the K and
 // V tiles staged in LDS serve all heads of the group (GQA) and every wave has a
 // full tile at every G (also when the rows are few).  Workgroup = (K split s,
 // chunk c, sequence b, kv head h).  A split is a range of split_tokens
@@ -27,8 +27,10 @@
 // split_tokens are finished by split 0, every other row's splits leave (max,
 // sum, unnormalised O) partials in the workspace for luc_prefill_merge.
 // Workgroups run longest first (split-major, the last chunk first), so short
-// ones fill the tail.  A workgroup walks its tokens in blocks of 64, grouped
-// into super-blocks (two blocks at head_dim 64, else one) in an LDS ring of NS
+// ones fill the tail.  The 4-wave workgroups (head_dim 64: half the LDS, two per CU, which
+// overlap one another's prologues; 128: one per CU) are for grids and contexts too
+// small to keep 8 waves busy, chosen by the host.  A workgroup walks its tokens in blocks of 64, grouped
+// into super-blocks (two blocks at head_dim 64 with 8 waves, else one) in an LDS ring of NS
 // stages (four at head_dim 64, three at 128): super-block J + NS - 2 loads
 // while super-block J is computed, and the waves meet at one barrier per
 // super-block.
@@ -225,11 +227,9 @@ __device__ constexpr uint32_t vslot(int t, int d) {
   return ((t >> 3) * (D / 32) + (d >> 5)) * 512 + ((t & 7) << 6) + (((d & 31) >> 2) << 3);
 }
 
-constexpr int kPrefillWaves = 8;
-
-template <int DT, int D>
+// W waves per workgroup, one 32-column tile each
+template <int DT, int D, int W>
 __device__ void prefill_impl(const PrefillArgs& A) {
-  constexpr int W = kPrefillWaves;  // waves per workgroup: one 32-column tile each
   constexpr int COLS = 32 * W;    // columns per chunk
   constexpr int BT = 64;          // tokens per block
   constexpr int CH = D / 8;       // 16-byte chunks per token row
@@ -237,8 +237,8 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   constexpr int KB = BT * ROWB;   // bytes of a K (or V) block
   // A stage holds SB consecutive blocks (a super-block): the waves meet at a
   // barrier once per stage.  Two blocks when the LDS of one workgroup per CU
-  // allows it (d64), else one.
-  constexpr int SB = D == 64 ? 2 : 1;
+  // allows it (d64, 8 waves), else one.
+  constexpr int SB = D == 64 && W == 8 ? 2 : 1;
   constexpr int KS = SB * KB;     // bytes of the K (or V) part of a stage
   constexpr int LOADS = KS / 1024;       // 1 KB wave-wide loads per K (or V) part
   constexpr int TPL = 1024 / ROWB;       // tokens per 1 KB load
@@ -248,7 +248,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   // t at slot c ^ kkey(t); V at vslot): super-block j is loaded NS - 2 stages
   // before its scores
   constexpr int NS = D == 64 ? 4 : 3;
-  constexpr bool PIPE = D == 64;  // the software-pipelined steps
+  constexpr bool PIPE = SB == 2;  // the software-pipelined steps
   constexpr int LPW = 2 * LOADS / W;  // loads per wave per stage
   static_assert(LOADS % W == 0, "every wave issues the same number of K (and V) loads");
   __shared__ __attribute__((aligned(16))) char s_kv[NS][2][KS];
@@ -423,7 +423,7 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   // stage tokens are page-aligned: token % page = load_token % page.  Kept
   // in registers except by the 8-wave head_dim 128 kernels, which have none
   // to spare (they recompute them)
-  constexpr bool KEEP_OFF = !(D == 128 && W == 8);
+  constexpr bool KEEP_OFF = D != 128 || W == 4;
   uint32_t lane_off[LPW];
 #pragma unroll
   for (int i = 0; i < LPW; ++i) lane_off[i] = KEEP_OFF ? load_offset(i, load_token(i, lane) % kPage, lane) : 0;
@@ -685,11 +685,55 @@ __device__ void prefill_impl(const PrefillArgs& A) {
     }
   };
   auto step = [&](int blk, f32x16* cur, f32x16* nxt) __attribute__((always_inline)) {
-    if (blk + 1 < nblk) {
-      boundary(blk);
-      if (blk + 1 < wblk) qk(blk + 1, nxt);
+    if constexpr (D == 64) {
+      // the LDS reads of K(blk + 1) and of the first half of V(blk) go out
+      // before the mask and max of block blk, the second half of V(blk)
+      // before its exponentials, so they land while the VALU works; the
+      // scores of blk + 1 reach the matrix cores before the exponentials,
+      // the PV of blk after them
+      if (blk + 1 < nblk) boundary(blk);
+      if (blk >= wblk) return;
+      u32x4_t ka[8];
+      u32x2_t va[16];
+      const bool has_next = blk + 1 < wblk;
+      if (has_next) {
+        const uint32_t kbase = lds_addr(s_kv[((blk + 1) / SB) % NS][0]) + ((blk + 1) % SB) * KB;
+        lds_k_issue<32 * ROWB>(kbase + krel[0], kbase + krel[1], kbase + krel[2], kbase + krel[3], ka);
+      }
+      const uint32_t vbase = lds_addr(s_kv[(blk / SB) % NS][1]) + (blk % SB) * KB;
+      lds_v_issue_half<ROWB, 0>(vbase + vrel[0], vbase + vrel[1], va);
+      softmax_max(blk, cur);
+      if (has_next) {
+        lds_wait_k<8>(ka);  // the first V reads of this block may still be in flight
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) nxt[hf][e] = 0.0f;
+#pragma unroll
+          for (int k = 0; k < NK; ++k)
+            nxt[hf] = mfma32<DT>(__builtin_bit_cast(uint4, ka[4 * hf + k]), qf[k], nxt[hf]);
+        }
+      }
+      lds_v_issue_half<ROWB, 1>(vbase + vrel[0], vbase + vrel[1], va);
+      softmax_exp(cur);
+      lds_wait_v(va);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint4 pb = p_operand(cur, c >> 1, c & 1);
+        osum = mfma32<DT>(ones, pb, osum);
+#pragma unroll
+        for (int db = 0; db < ND; ++db)
+          o[db] = mfma32<DT>(make_uint4(va[4 * c + 2 * db].x, va[4 * c + 2 * db].y,
+                                        va[4 * c + 2 * db + 1].x, va[4 * c + 2 * db + 1].y),
+                             pb, o[db]);
+      }
+    } else {
+      if (blk + 1 < nblk) {
+        boundary(blk);
+        if (blk + 1 < wblk) qk(blk + 1, nxt);
+      }
+      if (blk < wblk) softmax_pv(blk, cur);
     }
-    if (blk < wblk) softmax_pv(blk, cur);
   };
 
   if (threadIdx.x == 0) s_bad_tok = 0x7fffffff;  // (read by every wave only after a barrier below)
@@ -984,9 +1028,11 @@ __device__ void prefill_merge_impl(const PrefillArgs& A) {
 }  // namespace luc
 
 #define LUC_PREFILL(DTN, DT, D)                                                                 \
-  extern "C" __global__ __launch_bounds__(64 * luc::kPrefillWaves) void luc_prefill_##DTN##_d##D(    \
-      luc::PrefillArgs a) {                                                                     \
-    luc::prefill_impl<DT, D>(a);                                                                \
+  extern "C" __global__ __launch_bounds__(512) void luc_prefill_##DTN##_d##D(luc::PrefillArgs a) {   \
+    luc::prefill_impl<DT, D, 8>(a);                                                             \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(256, 2) void luc_prefill_##DTN##_d##D##_w4(luc::PrefillArgs a) { \
+    luc::prefill_impl<DT, D, 4>(a);                                                             \
   }                                                                                             \
   extern "C" __global__ __launch_bounds__(luc::kMergeThreads) void luc_prefill_merge_##DTN##_d##D(   \
       luc::PrefillArgs a) {                                                                     \

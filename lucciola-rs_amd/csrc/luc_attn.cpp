@@ -408,7 +408,7 @@ struct PrefillArgs {
   float qk_scale_log2;
 };
 
-// Prefill work split.  A workgroup takes a chunk of 256 (row, head of the
+// Prefill work split.  A workgroup takes a chunk of 256 (or 128) (row, head of the
 // group) columns of one (sequence, kv head) and one K split.  The lengths are on
 // the device: the plan takes `batch` sequences of equal rows that end at max_ctx,
 // which for one sequence is exact, and depends only on the arguments.
@@ -426,15 +426,33 @@ struct PrefillArgs {
 // 1024, 52.5 at 384, 59.5 whole; 700 rows of the same: 21.5 at 256, 22.7 at 128, 27.1
 // whole; 1000 rows, 12 and 2 of 128: 33.3 at 256, 39.1 at 128.
 //
+// Waves per workgroup of an unsplit launch (a split one: 8).  Workgroups of 4 waves
+// overlap one another's prologues at head_dim 64 (two per CU), and are twice as many
+// where 8-wave ones leave CUs idle; workgroups of 8 read K and V half as often.  us per
+// call on 8 waves and on 4:
+//   head_dim 64: 4 (256 prompts of 32 rows after 100, 16 and 16 heads: 134 and 85; 64 of
+//     500, 32 and 8 heads: 275 and 233; one of 2048, 32 and 8: 54 and 47; 4 of 2048, 64 and
+//     8: 238 and 222), but 8 where 4 give no more workgroups in the only round (16 of 100
+//     after 300, 16 and 16: 21.5 and 25.3) and for two to four rounds of long prompts
+//     at groups above 4 (4 of 2048, 14 and 2: 63.3 and 65.5; one of 2048, 64 and 8: 67.0
+//     and 68.6);
+//   head_dim 128 (one workgroup per CU either way; one of 4 waves takes 0.84 of the time
+//     for half the columns): 8, but 4 where 8-wave workgroups make at most one round
+//     and 4-wave ones end earlier (one of 2048, 32 and 8 heads: 92.8 and 86.3; 500 rows
+//     unsplit, 8 and 8: 29.2 and 24.6; not 2 of 950 after 2000, 28 and 4: 122 and 161).
+//
 // Grid.  Every (sequence, kv head) gets the chunks of the longest sequence the
 // arguments allow, min(total_rows, max_ctx) rows, or, where most of those would be idle
-// (more than 8 times the slots: 64 prompts of 128 rows after 4000, 64 and 8 heads of 128:
-// 1510 with the idle chunks, 1250 without), total_rows x group / columns + batch slots that the workgroups
-// deal among the sequences.  Short prompts of many sequences run in blocks of kPrefillBlock
-// (sequence, kv head) pairs, so that a pair's chunks run while its K and V are in L2 (64
-// prompts of 128 rows, 28 and 4 heads of 128: 81.3, in blocks 75.4).
-constexpr int kPrefillCols = 256;    // columns per workgroup: 8 waves x 32 (paged_prefill.hip)
+// (more than 4 times the slots), total_rows x group / columns + batch slots that the
+// workgroups deal among the sequences: us on chunks and on slots, 64 prompts of 128 rows, 64
+// and 8 heads of 128, after 500 positions (4 times): 334 and 325, after 1000 486 and 457,
+// after 4000 1510 and 1250; 128 of 40 rows after 200, 32 and 8 of 64 (3.5 times): 58.8 and 59.2,
+// after 400 77.4 and 75.2.  Short prompts of many sequences run in blocks of
+// kPrefillBlock (sequence, kv head) pairs, so that a pair's chunks run while its K and
+// V are in L2 (64 prompts of 128 rows, 28 and 4 heads of 128: 81.3, in blocks 75.4).
+constexpr int kPrefillCols = 256;    // columns per 8-wave workgroup: 8 x 32 (paged_prefill.hip)
 struct PrefillPlan {
+  int waves = 8;
   int chunks = 0;  // per (sequence, kv head), at most
   int slots = 0;   // per kv head, instead
   int gblock = 0;  // (sequence, kv head) pairs per block
@@ -448,7 +466,7 @@ constexpr int kMaxPrefillSplits = 64;
 constexpr int kPrefillBlock = 64;
 constexpr int kMaxGridYZ = 65535;
 constexpr int kMaxSlotSeqs = 512;  // (a workgroup reads the lengths of 64 sequences at a time)
-PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_ctx,
+PrefillPlan prefill_plan(int batch, int hkv, int group, int head_dim, int total_rows, int max_ctx,
                          bool may_split) {
   PrefillPlan p;
   const int64_t rows = std::min(total_rows, max_ctx);
@@ -496,10 +514,27 @@ PrefillPlan prefill_plan(int batch, int hkv, int group, int total_rows, int max_
       tokens -= step;
     }
   }
-  const int64_t chunks = ceil_div(rows * group, kPrefillCols);
-  const int64_t slots = (int64_t)total_rows * group / kPrefillCols + batch;
-  if ((batch <= kMaxSlotSeqs && batch * chunks > 8 * slots) || chunks > kMaxGridYZ ||
-      groups * chunks * (2 * kPrefillCols) > UINT32_MAX) {
+  if (p.splits == 1) {
+    const int64_t wgs8 = n * groups, wgs4 = ceil_div(seq_rows * group, kPrefillCols / 2) * groups;
+    const int64_t rounds = ceil_div(wgs8, kPrefillSlots);
+    bool four;
+    if (head_dim == 64) {
+      four = rounds == 1 ? wgs4 > wgs8 : group <= 4 || rounds > 4 || max_ctx <= 1024 || max_ctx >= 4 * seq_rows;
+    } else {
+      // two workgroups after one another on the CU that ends last: the longest first,
+      // at most the contexts of ranks kPrefillSlots and the next (they fall linearly from max_ctx)
+      const int64_t unit = 64 * kPrefillUnit;
+      const int64_t pair = wgs4 <= kPrefillSlots ? 0
+                           : 2 * (max_ctx - seq_rows * kPrefillSlots / wgs4 + unit);
+      four = rounds == 1 && wgs4 > wgs8 && pair * 84 < (max_ctx + unit) * 100;
+    }
+    p.waves = four ? 4 : 8;
+  }
+  const int cols = 32 * p.waves;
+  const int64_t chunks = ceil_div(rows * group, cols);
+  const int64_t slots = (int64_t)total_rows * group / cols + batch;
+  if ((batch <= kMaxSlotSeqs && batch * chunks > 4 * slots) || chunks > kMaxGridYZ ||
+      groups * chunks * (64 * p.waves) > UINT32_MAX) {
     p.slots = (int)std::min<int64_t>(slots, INT32_MAX);
   } else {
     p.chunks = (int)chunks;
@@ -597,6 +632,7 @@ int luc_init(int device, const char* code_object_dir, luc_ctx** out_ctx) {
     for (int d : {64, 128})
       for (const char* kind : {"luc_prefill_", "luc_prefill_merge_"})
         names.push_back(std::string(kind) + dt + "_d" + std::to_string(d));
+    for (int d : {64, 128}) names.push_back(std::string("luc_prefill_") + dt + "_d" + std::to_string(d) + "_w4");
     for (int d : {64, 128})
       for (int g = 1; g <= 8; ++g)
         for (const char* kind : {"luc_decode_", "luc_decode_step_"}) {
@@ -839,7 +875,7 @@ static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64
     return fail(LUC_E_INVALID, "table_stride %d pages cannot hold max_ctx %d", table_stride, max_ctx);
   if (batch == 0 || total_rows == 0) return LUC_OK;
   const int group = num_q_heads / num_kv_heads;
-  const PrefillPlan plan = prefill_plan(batch, num_kv_heads, group, total_rows, max_ctx, split);
+  const PrefillPlan plan = prefill_plan(batch, num_kv_heads, group, head_dim, total_rows, max_ctx, split);
   const size_t need = prefill_workspace_bytes(plan, total_rows, num_q_heads, head_dim);
   if (need && (!workspace || workspace_bytes < need))
     return fail(LUC_E_WORKSPACE, "workspace %zu bytes, %zu needed", workspace_bytes, need);
@@ -847,13 +883,13 @@ static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64
   if (int rc = check_device(ctx)) return rc;
   const std::string suffix = std::string(dt_name(dtype)) + "_d" + std::to_string(head_dim);
   hipFunction_t fn, merge;
-  if (int rc = get_fn(ctx, "luc_prefill_" + suffix, &fn)) return rc;
+  if (int rc = get_fn(ctx, "luc_prefill_" + suffix + (plan.waves == 4 ? "_w4" : ""), &fn)) return rc;
   if (int rc = get_fn(ctx, "luc_prefill_merge_" + suffix, &merge)) return rc;
   // slots: (slot and kv head, 1, split); else (pairs of a block, chunk, split or block)
   const int64_t pairs = (int64_t)batch * num_kv_heads;
   const int64_t grid_x = plan.slots ? (int64_t)plan.slots * num_kv_heads : plan.gblock;
   const int64_t grid_z = plan.slots || plan.splits > 1 ? plan.splits : ceil_div(pairs, plan.gblock);
-  if (grid_x * 2 * kPrefillCols > UINT32_MAX || grid_z > kMaxGridYZ)
+  if (grid_x * 64 * plan.waves > UINT32_MAX || grid_z > kMaxGridYZ)
     return fail(LUC_E_INVALID, "batch x kv heads x row tiles too large");
   const dim3 grid((unsigned)grid_x, (unsigned)std::max(plan.chunks, 1), (unsigned)grid_z);
 
@@ -892,7 +928,7 @@ static int paged_prefill(luc_ctx* ctx, void* stream, int dtype, void* qkv, int64
                                       prefill_ml_bytes(plan, total_rows, num_q_heads));
   }
   void* args[] = {&p};
-  if (int rc = launch(fn, grid, dim3(2 * kPrefillCols), stream, args)) return rc;
+  if (int rc = launch(fn, grid, dim3(64 * plan.waves), stream, args)) return rc;
   if (!need) return LUC_OK;
   // 3) the rows that several splits share (head_dim / 4 lanes per row and head)
   const int64_t items = (int64_t)total_rows * num_q_heads;
@@ -919,7 +955,7 @@ size_t luc_paged_prefill_workspace_size(int batch, int total_rows, int max_ctx, 
       num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > 8 || (head_dim != 64 && head_dim != 128))
     return 0;
   return prefill_workspace_bytes(
-      prefill_plan(batch, num_kv_heads, num_q_heads / num_kv_heads, total_rows, max_ctx, true),
+      prefill_plan(batch, num_kv_heads, num_q_heads / num_kv_heads, head_dim, total_rows, max_ctx, true),
       total_rows, num_q_heads, head_dim);
 }
 

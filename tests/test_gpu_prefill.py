@@ -2,6 +2,8 @@
 vs the oracle, through the C ABI.  Roped q/k (in place) and the cache are
 compared bit for bit; attention outputs within the stated tolerance
 (max-abs 2e-3 fp16, 1e-2 bf16)."""
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -272,3 +274,32 @@ def test_prefill_many_prompts_under_a_long_bound(orc, luc):
     assert torch.isfinite(results[0][1]).all() and results[0][1].any(-1).all()
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@contextlib.contextmanager
+def unsplit(luc):
+    """luc_paged_prefill, which cuts no contexts, in the place of luc_paged_prefill_split."""
+    size, split = luc.lib.luc_paged_prefill_workspace_size, luc.lib.luc_paged_prefill_split
+    try:
+        luc.lib.luc_paged_prefill_workspace_size = lambda *a: 0
+        luc.lib.luc_paged_prefill_split = lambda *a: luc.lib.luc_paged_prefill(*a[:-2])
+        yield
+    finally:
+        luc.lib.luc_paged_prefill_workspace_size, luc.lib.luc_paged_prefill_split = size, split
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 4, 64), (14, 2, 64), (8, 8, 128), (12, 2, 128), (32, 4, 128)])
+def test_prefill_unsplit_at_chunk_edges(orc, luc, hq, hkv, d, dtype):
+    """Whole contexts, as luc_paged_prefill takes them, on 4-wave workgroups (so few
+    rows leave CUs idle): prompts that end one column of a 128-column chunk
+    before its end, on it and past it (where the group size divides it), after
+    prefixes that end on and around a 64-token block, with biases, in layer 2 of 3."""
+    g = hq // hkv
+    cfg = wl.PrefillConfig("edges", 4, 0, hq, hkv, d, dtype, 0, 0, 0.5)
+    h = wl.host_prefill_inputs(cfg, seed=hq + d, num_layers=3, starts=[0, 63, 64, 130],
+                               rows=[128 // g, 256 // g + 1, 128 // g - 1, 3])
+    bias = biases(cfg, 13)
+    with unsplit(luc):
+        got = gpu_prefill(luc, h, layer=2, bias=bias)
+    assert_prefill_matches(orc, got, oracle_prefill(orc, luc, h, layer=2, bias=bias), dtype)
