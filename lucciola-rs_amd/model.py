@@ -12,8 +12,8 @@ Per layer (Qwen2Model::forward_layer, models.rs:434-691):
   gu     = norm @ gate_up_proj^T                        GEMM
   gate   = silu(gate) * up                              luc_silu_mul
   h      = gate @ down_proj^T + h                       GEMM, beta = 1
-For a prompt whose sizes fit them, luc_prompt_gemm is the q/k/v product and
-luc_prompt_mlp everything from o to the next layer's norm.
+For a prompt whose sizes fit them (prompt_kernels_win), luc_prompt_gemm is the
+q/k/v product and luc_prompt_mlp everything from o to the next layer's norm.
 For one row (a decode step) the products are GEMVs with the norms and silu * up
 fused into them, five launches a layer with the same bits as the unfused ones:
 luc_rmsnorm_gemv (q/k/v), luc_decode_step, luc_gemv (o, + h),
@@ -107,15 +107,38 @@ def _dev(bits: np.ndarray, device) -> torch.Tensor:
 
 GEMV_MAX_K = 8192  # the longest weight row luc_gemv / luc_rmsnorm_gemv / luc_gate_up_silu take
 
+# luc_prompt_gemm and luc_prompt_mlp against hipBLASLt with separate norm and silu launches,
+# us a layer (queueing included), up to this many rows and multiply-adds of the products:
+#   hidden 896, intermediate 4864: 38 and 97 at 64 rows, 67 and 98 at 700, 103 and 109 at
+#     1300, 139 and 143 at 2048, 234 and 203 at 4096;
+#   1024, 2816: 86 and 108 at 1100 rows, 110 and 106 at 1537;
+#   1536, 8960: 145 and 138 at 700 (181 on transposed copies), 235 and 192 at 1281;
+#   3584, 18944: 146 and 203 at 64, 242 and 275 at 200, 555 and 425 at 700;
+#   5120, 13824: 155 and 165 at 64, 310 and 244 at 193 (343 on copies), 1535 and 989 at 2000;
+#   8192, 28672: 384 and 407 at 64, 741 and 657 at 200, 4212 and 2423 at 2000.
+# The library's tiles reach twice the rate where the rows fill the chip; these kernels
+# save its launches and passes where they do not.
+PROMPT_KERNEL_ROWS = 1536
+PROMPT_KERNEL_WORK = 50_000_000_000
+
+
+def prompt_kernels_win(cfg: Qwen2Config, rows: int) -> bool:
+    """Whether a prompt of `rows` rows runs on luc_prompt_gemm and luc_prompt_mlp
+    (their sizes allow it and they are the faster ones) or on library GEMMs."""
+    H, I = cfg.hidden_size, cfg.intermediate_size
+    if H % 64 or I % 64:
+        return False
+    return rows <= PROMPT_KERNEL_ROWS and rows * H * (cfg.qkv_dim + H + 3 * I) <= PROMPT_KERNEL_WORK
+
 
 class Qwen2Model:
     """One sequence through the decoder: `forward(ids, cache_pos)` then
     `sample_greedy()`, or `generate` (models.rs:184-243).  The products of a
     single row (every decode step) are luc_gemv on the weights in the
     reference's [out, in] layout ("*_w"); those of a prompt are the MFMA products
-    of luc_prompt_gemm and luc_prompt_mlp on the same weights, or, for sizes that
-    these do not take (hidden or intermediate not a multiple of 64), hipBLASLt
-    GEMMs on a transposed copy ([in, out], contiguous: "*_t")."""
+    of luc_prompt_gemm and luc_prompt_mlp on the same weights, or, where
+    prompt_kernels_win says so, hipBLASLt GEMMs on their transposes ("*_t": views,
+    or contiguous copies where hidden or intermediate is not a multiple of 64)."""
 
     def __init__(self, cfg: Qwen2Config, weights: dict, num_blocks: int | None = None,
                  max_positions: int | None = None, device="cuda", lib=None):
@@ -129,7 +152,7 @@ class Qwen2Model:
         if cfg.hidden_size % cfg.num_attention_heads or d not in (64, 128):
             raise ValueError(f"unsupported head_dim {d}")
         H, I = cfg.hidden_size, cfg.intermediate_size
-        self.prompt_kernels = H % 64 == 0 and I % 64 == 0
+        views = H % 64 == 0 and I % 64 == 0
         self.embed = _dev(weights["embed_tokens"], self.device)
         # [vocab, hidden] for the one-row logits: the embedding when tied
         self.lm_head_w = _dev(weights["lm_head"], self.device) if "lm_head" in weights else self.embed
@@ -148,11 +171,11 @@ class Qwen2Model:
                 "gate_up_w": W("gate_up_proj"),
                 "down_w": W("down_proj"),
             }
-            if not self.prompt_kernels:
-                for name in ("qkv", "o", "gate_up"):
-                    L[name + "_t"] = L[name + "_w"].t().contiguous()
-            if not self.prompt_kernels or I > GEMV_MAX_K:  # (one row: _layer)
-                L["down_t"] = L["down_w"].t().contiguous()
+            for name in ("qkv", "o", "gate_up", "down"):
+                wt = L[name + "_w"].t()
+                L[name + "_t"] = wt if views else wt.contiguous()
+            if I > GEMV_MAX_K:  # (one row: _layer)
+                L["down_row"] = L["down_t"].contiguous()
             self.layers.append(L)
         max_pos = max_positions or cfg.max_position_embeddings
         self.max_positions = max_pos
@@ -220,7 +243,7 @@ class Qwen2Model:
                 self.lib.gemv(y, act, L["down_w"], residual=h)
                 return y
             # rows longer than the GEMV takes (Qwen2-1.5B's 8960): a GEMM
-            h.addmm_(act, L["down_t"])
+            h.addmm_(act, L["down_row"])
             if out is None:
                 return h
             out.copy_(h)
@@ -279,7 +302,7 @@ class Qwen2Model:
             start = torch.tensor([cache_pos], dtype=torch.int32, device=self.device)
             attention = lambda li, qkv: self._attention_prefill(li, qkv, cache_pos, cu, start)  # noqa: E731
         n = cfg.num_hidden_layers
-        if S > 1 and self.prompt_kernels:
+        if S > 1 and prompt_kernels_win(cfg, S):
             self._prompt_layers(h, attention)
             self.hidden.copy_(h[S - 1:])
             return

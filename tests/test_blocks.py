@@ -189,3 +189,32 @@ def test_model_reserves_the_pages_of_every_position(calls):
         pages = -(-last // 16)
         assert m.kv.block_table_cpu == list(range(pages))
         assert lib.tables[-1].reshape(-1)[:pages].tolist() == list(range(pages))
+
+
+@pytest.mark.parametrize("hidden,heads,kv,inter,kernels,library", [
+    (896, 14, 2, 4864, 700, 2500), (896, 14, 2, 4864, 1536, 4096), (1024, 16, 16, 2816, 1100, 2048),
+    (1536, 12, 2, 8960, 700, 1281), (2048, 16, 2, 11008, 300, 769), (3584, 28, 4, 18944, 129, 700),
+    (5120, 40, 8, 13824, 64, 257), (8192, 64, 8, 28672, 16, 200), (896, 14, 2, 4872, None, 5)])
+def test_prompt_products_rule(hidden, heads, kv, inter, kernels, library):
+    """Prompts run on the library GEMMs where these measured faster (large row
+    counts and widths; sizes the kernels do not take), and on this library's own
+    products elsewhere."""
+    cfg = dataclasses.replace(model.QWEN25_05B, hidden_size=hidden, num_attention_heads=heads,
+                              num_key_value_heads=kv, intermediate_size=inter)
+    assert kernels is None or model.prompt_kernels_win(cfg, kernels)
+    assert not model.prompt_kernels_win(cfg, library)
+
+
+@pytest.mark.parametrize("rows,own", [(2, 1), (1536, 1), (1537, 0)])
+def test_model_prompt_follows_the_rule(rows, own):
+    """Qwen2Model.forward launches luc_prompt_gemm once a layer where the rule
+    says so, and not at all elsewhere."""
+    cfg = dataclasses.replace(model.QWEN25_05B, hidden_size=128, intermediate_size=128,
+                              num_attention_heads=2, num_key_value_heads=1, num_hidden_layers=2,
+                              vocab_size=64)
+    lib = _NoLaunch()
+    calls = []
+    lib.prompt_gemm = lambda *a: calls.append(a[1].shape[0])
+    m = model.Qwen2Model(cfg, model.random_weights(cfg, 0), max_positions=2048, device="cpu", lib=lib)
+    m.forward([1] * rows, 0)
+    assert calls == [rows] * 2 * own

@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 import torch
 
-from lucciola_rs_amd.model import QWEN25_05B, Qwen2Model, random_weights, to_bf16_bits
+from lucciola_rs_amd import model as model_module
+from lucciola_rs_amd.model import QWEN25_05B, Qwen2Config, Qwen2Model, random_weights, to_bf16_bits
 from gpu_util import from_dev, say, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -635,3 +636,29 @@ def test_prompt_layer_products(luc, rows, hidden, inter):
         say(f"  {name}: max {float(d.max()):.3e}, beyond a unit {over:.4f}")
         assert float((d / want.abs().amax(-1, keepdim=True)).max()) <= 2 ** -7, name
         assert over <= 1 / 64, name
+
+
+@pytest.mark.parametrize("inter", [320, 8320])
+def test_prompt_products_agree_with_library_gemms(luc, monkeypatch, inter):
+    """A prompt through luc_prompt_gemm / luc_prompt_mlp and through the library
+    GEMMs on the same weights: both sum in f32 and round to bf16 at the same
+    places, so they differ by the units that another sum order moves.  A row's
+    relative error from one such rounding is at most 2^-9 in the 2-norm; a layer
+    has seven (norm, q/k/v, attention, h, norm, gate and up, act) before the
+    last h, two layers fourteen, and independent ones add as squares: sqrt(14) 2^-9
+    = 0.0073, doubled for two paths that round apart."""
+    cfg = Qwen2Config(vocab_size=512, hidden_size=256, num_hidden_layers=2, num_attention_heads=4,
+                      num_key_value_heads=2, intermediate_size=inter, max_position_embeddings=512)
+    w = random_weights(cfg, 5, std=0.06)
+    ids = [int(i) for i in np.random.default_rng(6).integers(0, 512, 130)]
+    got = []
+    for rows in (model_module.PROMPT_KERNEL_ROWS, 0):
+        monkeypatch.setattr(model_module, "PROMPT_KERNEL_ROWS", rows)
+        m = Qwen2Model(cfg, w, max_positions=256, lib=luc)
+        m.forward(ids, 0)
+        got.append([t.float() for t in (m.hidden, m.logits(), m.kv.k_pool, m.kv.v_pool)])
+    torch.cuda.synchronize()
+    for a, b in zip(*got):
+        err = float((a - b).norm() / b.norm())
+        say(f"  own products against library GEMMs: {err:.2e}")
+        assert err <= 2 * 14 ** 0.5 * 2 ** -9
