@@ -23,7 +23,8 @@ def biases(cfg, seed):
             wl.to_bits(wl.normal(rng, (cfg.hkv * d,), 0.5), cfg.dtype))
 
 
-def gpu_prefill(luc, h: wl.HostPrefill, layer=0, max_ctx=None, bias=None):
+def gpu_prefill(luc, h: wl.HostPrefill, layer=0, max_ctx=None, bias=None, scale=None, stream=None,
+                num_blocks=None):
     cfg = h.cfg
     d = cfg.head_dim
     rope = rope_cache(luc, d)
@@ -39,22 +40,25 @@ def gpu_prefill(luc, h: wl.HostPrefill, layer=0, max_ctx=None, bias=None):
     say(f"  [gpu] paged_prefill {cfg.name} rows={np.diff(h.cu_seqlens).tolist()[:8]} "
         f"starts={h.start_pos.tolist()[:8]} hq={cfg.hq} hkv={cfg.hkv} d={d} {cfg.dtype} "
         f"max_ctx={max_ctx} layer={layer} bias={bias is not None}")
+    if stream is not None:
+        stream.wait_stream(torch.cuda.current_stream())
     luc.paged_prefill(qkv, qb, kb, vb, rope.cos, rope.sin, kp, vp, tables, cu, sp, total, max_ctx,
-                      layer, h.num_layers, cfg.hq, cfg.hkv, d, sm_scale(d), out)
+                      layer, h.num_layers, cfg.hq, cfg.hkv, d, sm_scale(d) if scale is None else scale,
+                      out, stream=stream, num_blocks=num_blocks)
     torch.cuda.synchronize()
     return dict(out=from_dev(out).reshape(total, cfg.hq, d), qkv=from_dev(qkv),
                 k_pool=from_dev(kp), v_pool=from_dev(vp))
 
 
-def oracle_prefill(orc, luc, h: wl.HostPrefill, layer=0, bias=None):
+def oracle_prefill(orc, luc, h: wl.HostPrefill, layer=0, bias=None, scale=None):
     cfg = h.cfg
     rope = rope_cache(luc, cfg.head_dim)
     cos, sin = rope.cos.cpu().numpy(), rope.sin.cpu().numpy()
     qkv, kp, vp = h.qkv.copy(), h.k_pool.copy(), h.v_pool.copy()
     qb, kb, vb = (None, None, None) if bias is None else bias
     out = orc.prefill(qkv, qb, kb, vb, cos, sin, kp, vp, h.tables, h.cu_seqlens, h.start_pos,
-                      layer, cfg.hq, cfg.hkv, cfg.head_dim, sm_scale(cfg.head_dim), 16,
-                      h.num_layers, cfg.dtype)
+                      layer, cfg.hq, cfg.hkv, cfg.head_dim,
+                      sm_scale(cfg.head_dim) if scale is None else scale, 16, h.num_layers, cfg.dtype)
     return dict(out=out, qkv=qkv, k_pool=kp, v_pool=vp)
 
 
@@ -303,3 +307,67 @@ def test_prefill_unsplit_at_chunk_edges(orc, luc, hq, hkv, d, dtype):
     with unsplit(luc):
         got = gpu_prefill(luc, h, layer=2, bias=bias)
     assert_prefill_matches(orc, got, oracle_prefill(orc, luc, h, layer=2, bias=bias), dtype)
+
+
+def split_prefill(hq, hkv, d, dtype, rows, starts, seed, luc, max_ctx=None, **kw):
+    """Inputs whose contexts the plan cuts."""
+    cfg = wl.PrefillConfig("split", len(rows), 0, hq, hkv, d, dtype, 0, 0, 0.5)
+    h = wl.host_prefill_inputs(cfg, seed=seed, rows=rows, starts=starts, **kw)
+    need = luc.lib.luc_paged_prefill_workspace_size(len(rows), int(h.cu_seqlens[-1]),
+                                                    max_ctx or h.max_ctx, hq, hkv, d)
+    assert need > 0, "these sizes are meant to split"
+    return h
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (12, 2, 128)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_prefill_split_with_biases_and_layer(orc, luc, hq, hkv, d, dtype, sign):
+    """Cut contexts with q, k and v biases, in layers 0 and 2 of 3, in both dtypes and
+    with a negative score scale, on a stream of its own (whose workspace the wrapper
+    allocates there) while the current one is another."""
+    h = split_prefill(hq, hkv, d, dtype, [300, 1, 90], [600, 880, 0], 31, luc, num_layers=3)
+    bias = biases(h.cfg, 32)
+    stream = torch.cuda.Stream()
+    for layer in (0, 2):
+        want = oracle_prefill(orc, luc, h, layer=layer, bias=bias, scale=sign * sm_scale(d))
+        assert_prefill_matches(orc, gpu_prefill(luc, h, layer=layer, bias=bias, scale=sign * sm_scale(d)),
+                               want, dtype)
+        got = gpu_prefill(luc, h, layer=layer, bias=bias, scale=sign * sm_scale(d), stream=stream)
+        assert_prefill_matches(orc, got, want, dtype)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (12, 2, 128)])
+def test_prefill_split_page_outside_the_pool(orc, luc, hq, hkv, d):
+    """A table entry outside the pool that only one split of several sees (tokens
+    640..655 of 900): the rows before it match the oracle, the rows at and after it
+    are NaN, in that split and in the next, and the other sequence is untouched."""
+    h = split_prefill(hq, hkv, d, "bf16", [300, 90], [600, 700], 33, luc, poison=False)
+    want = oracle_prefill(orc, luc, h)
+    tables = h.tables.copy()
+    tables[0, 40] = h.k_pool.shape[0] + 1
+    spare = np.zeros((4,) + h.k_pool.shape[1:], np.uint16)
+    bad = wl.replace(h, tables=tables, k_pool=np.concatenate([h.k_pool, spare]),
+                     v_pool=np.concatenate([h.v_pool, spare]))
+    got = gpu_prefill(luc, bad, num_blocks=h.k_pool.shape[0])
+    o, w = orc.to_f32(got["out"], "bf16"), orc.to_f32(want["out"], "bf16")
+    ok = np.r_[np.arange(300) < 40, np.ones(90, bool)]
+    assert np.all(np.isnan(o[~ok]))
+    assert np.max(np.abs(o[ok] - w[ok])) <= TOL["bf16"]
+    assert not got["k_pool"][-4:].any() and not got["v_pool"][-4:].any()
+    assert np.array_equal(got["qkv"], want["qkv"])
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (12, 2, 128)])
+def test_prefill_split_beside_a_flagged_sequence(orc, luc, hq, hkv, d):
+    """A sequence past max_ctx between two whose contexts are cut: NaN in all of its
+    rows (and no later split or merge writes there), the oracle's results in theirs."""
+    h = split_prefill(hq, hkv, d, "bf16", [200, 50, 100], [600, 1200, 650], 34, luc, max_ctx=800)
+    got = gpu_prefill(luc, h, max_ctx=800)
+    want = oracle_prefill(orc, luc, h)
+    o, w = orc.to_f32(got["out"], "bf16"), orc.to_f32(want["out"], "bf16")
+    assert np.all(np.isnan(o[200:250]))
+    for rows in (slice(0, 200), slice(250, 350)):
+        assert np.max(np.abs(o[rows] - w[rows])) <= TOL["bf16"]
+    for name in ("qkv", "k_pool", "v_pool"):
+        assert np.array_equal(got[name], want[name]), name
