@@ -262,8 +262,8 @@ __device__ void prefill_impl(const PrefillArgs& A) {
   int b, h, split, chunk = 0, nchunks = 0;
   if (A.slots) {
     // grid (slot x kv head, 1, split): the chunks of sequence 0, then those of
-    // sequence 1, ..., and unused slots at the end (spread among the others they
-    // would leave some shader engines without work)
+    // sequence 1, ..., and unused slots at the end (64 prompts of 128 rows after 4000,
+    // 16 and 8 heads of 128: 371 us; with every second slot unused 620)
     const int slot = blockIdx.x / A.hkv;
     h = blockIdx.x - slot * A.hkv;
     split = blockIdx.z;

@@ -22,7 +22,8 @@
 // bank.  W is the MFMA's A operand and x its B operand: a lane then holds 4
 // consecutive columns of one row of y.
 //
-// What bounds it: at these sizes a workgroup runs 14 to 76 steps, each a barrier, LDS reads and
+// What bounds it (hidden 896, intermediate 4864): a workgroup runs 14 steps (q/k/v, gate/up),
+// 4 to 7 (o, in K ranges) or 4 to 38 (down), each a barrier, LDS reads and
 // loads from L2 (8 to 10 TB/s in all); larger tiles halve the reads and loads per
 // MFMA and win once the rows fill the chip with them (us, hidden 896, intermediate
 // 4864): gate/up 28.7 on 64-row tiles and 24.1 on 128 at 700 rows, 15.7 and 16.1 at
@@ -33,7 +34,7 @@
 // 19.2, the two reductions with their norms 4.7 each; hipBLASLt with separate norm and
 // silu kernels took 11.5, 11.5, 23.3 + 6.3, 28.5 and 3.9 each, with ten launches a layer queued from Python.
 //
-// A prompt's rows are few (5 to some thousand), so the tiles are small to fill 256
+// They are for prompts of few rows (5 to 1500), so the tiles are small to fill 256
 // CUs, and o and down, with N = hidden, are split over K as well.  The tiles of a W row
 // block go to one XCD (workgroup id mod 8), so W is read from HBM once and x
 // (which fits every XCD's L2) by all.  Rows and columns past the end re-read the

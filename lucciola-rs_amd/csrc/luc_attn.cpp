@@ -1089,9 +1089,10 @@ struct GemmArgs {
   void* y;
   int32_t m, n, k, splits, m_tiles, n_tiles;
 };
-// Tiles of 128 rows where the rows fill the chip with them (prompt_gemm.hip,
-// measured there): the gate/up pairs (38 row blocks of W and more) from 257 rows on, o and
-// down (128 x 128 tiles, a seventh of the workgroups) from 1024.
+// Tiles of 128 rows from the row counts on where they were the faster ones at hidden 896 and
+// intermediate 4864 (prompt_gemm.hip): the gate/up pairs (76 row blocks of W) from 257, o
+// and down (128 x 128 tiles, a seventh of the workgroups) from 1024.  Wider layers fill the
+// chip, and leave these products for a library's, at fewer rows (Qwen2Model's rule).
 int gemm_tile_rows(bool silu, int rows) { return rows >= (silu ? 257 : 1024) ? 128 : 64; }
 // K ranges of a split product: as many as keep an XCD's workgroups (its share of
 // the W row blocks, 8 apart, x row tiles x ranges) in one round of two per CU, each of at

@@ -438,8 +438,8 @@ def test_greedy_after_2048_token_prefill(orc):
 def test_greedy_lockstep_full_oracle(orc, qwen):
     """End to end against the oracle's whole loop (oracle/model.py, its GEMMs
     on the host BLAS): a 32-token prompt, then 128 steps teacher-forced by the
-    oracle's greedy token.  The GEMMs' summation orders differ (hipBLASLt
-    here, BLAS in the oracle, cuBLAS in the reference), so where the two
+    oracle's greedy token.  The GEMMs' summation orders differ
+    (luc_prompt_gemm here, BLAS in the oracle, cuBLAS in the reference), so where the two
     greedy tokens differ the step must be a near-tie: the GPU's token within
     that step's largest logit difference of the oracle's best.  At least 90%
     of the steps must agree."""
