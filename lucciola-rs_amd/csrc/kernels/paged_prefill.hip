@@ -22,7 +22,7 @@
 // chunk c, sequence b, kv head h).  A split is a range of split_tokens
 // positions; the host cuts the contexts where the chunks alone leave CUs idle
 // (512 rows after 8000 cached, 12 q- and 2 kv-heads of 128: 24 chunks, 54 us a
-// call in 10 splits, 284 with every context whole).
+// call in 10 splits, 243 with every context whole).
 // Row i's position falls into the last split it reads: rows of positions below
 // split_tokens are finished by split 0, every other row's splits leave (max,
 // sum, unnormalised O) partials in the workspace for luc_prefill_merge.

@@ -420,7 +420,7 @@ struct PrefillArgs {
 // mean load of a CU plus half a workgroup of tail; and a split launch pays
 // kPrefillMerge and, for every split, 3/4 of a block of partials written and merged.
 // Measured against fixed lengths (us per call): 512 rows after 8000, 12 and 2 heads of 128:
-// 56.3 at the plan's 896 tokens, 73.7 at 768 (264 workgroups), 57.6 at 1024, 284 whole;
+// 56.3 at the plan's 896 tokens, 73.7 at 768 (264 workgroups), 57.6 at 1024, 284 whole (on 8 waves);
 // 128 rows after 2000, 14 and 2 of 64: 22.8 at the plan's 384, 22.2 at
 // 256, 24.3 at 128, 24.6 at 512, 50 whole; 2500 rows of the same: 41.8 at
 // 1024, 52.5 at 384, 59.5 whole; 700 rows of the same: 21.5 at 256, 22.7 at 128, 27.1

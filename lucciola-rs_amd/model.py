@@ -108,7 +108,10 @@ def _dev(bits: np.ndarray, device) -> torch.Tensor:
 GEMV_MAX_K = 8192  # the longest weight row luc_gemv / luc_rmsnorm_gemv / luc_gate_up_silu take
 
 # luc_prompt_gemm and luc_prompt_mlp against hipBLASLt with separate norm and silu launches,
-# us a layer (queueing included), up to this many rows and multiply-adds of the products:
+# us a layer (queueing included), up to this many rows and multiply-adds of the products, or
+# where those are few (the library's launches are then most of its time):
+#   hidden 256, intermediate 704: 77 and 103 at 6000 rows; 512, 1408: 92 and 103 at 4096,
+#     121 and 106 at 6000; 768, 3072: 92 and 104 at 1537, 120 and 115 at 2600;
 #   hidden 896, intermediate 4864: 38 and 97 at 64 rows, 67 and 98 at 700, 103 and 109 at
 #     1300, 139 and 143 at 2048, 234 and 203 at 4096;
 #   1024, 2816: 86 and 108 at 1100 rows, 110 and 106 at 1537;
@@ -120,6 +123,7 @@ GEMV_MAX_K = 8192  # the longest weight row luc_gemv / luc_rmsnorm_gemv / luc_ga
 # save its launches and passes where they do not.
 PROMPT_KERNEL_ROWS = 1536
 PROMPT_KERNEL_WORK = 50_000_000_000
+PROMPT_KERNEL_FEW = 15_000_000_000
 
 
 def prompt_kernels_win(cfg: Qwen2Config, rows: int) -> bool:
@@ -128,7 +132,8 @@ def prompt_kernels_win(cfg: Qwen2Config, rows: int) -> bool:
     H, I = cfg.hidden_size, cfg.intermediate_size
     if H % 64 or I % 64:
         return False
-    return rows <= PROMPT_KERNEL_ROWS and rows * H * (cfg.qkv_dim + H + 3 * I) <= PROMPT_KERNEL_WORK
+    work = rows * H * (cfg.qkv_dim + H + 3 * I)
+    return work <= (PROMPT_KERNEL_WORK if rows <= PROMPT_KERNEL_ROWS else PROMPT_KERNEL_FEW)
 
 
 class Qwen2Model:

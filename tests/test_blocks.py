@@ -192,7 +192,7 @@ def test_model_reserves_the_pages_of_every_position(calls):
 
 
 @pytest.mark.parametrize("hidden,heads,kv,inter,kernels,library", [
-    (896, 14, 2, 4864, 700, 2500), (896, 14, 2, 4864, 1536, 4096), (1024, 16, 16, 2816, 1100, 2048),
+    (256, 4, 2, 704, 6000, 30000), (512, 8, 2, 1408, 4096, 6000), (896, 14, 2, 4864, 700, 2500), (896, 14, 2, 4864, 1536, 4096), (1024, 16, 16, 2816, 1100, 2048),
     (1536, 12, 2, 8960, 700, 1281), (2048, 16, 2, 11008, 300, 769), (3584, 28, 4, 18944, 129, 700),
     (5120, 40, 8, 13824, 64, 257), (8192, 64, 8, 28672, 16, 200), (896, 14, 2, 4872, None, 5)])
 def test_prompt_products_rule(hidden, heads, kv, inter, kernels, library):
@@ -206,12 +206,13 @@ def test_prompt_products_rule(hidden, heads, kv, inter, kernels, library):
 
 
 @pytest.mark.parametrize("rows,own", [(2, 1), (1536, 1), (1537, 0)])
-def test_model_prompt_follows_the_rule(rows, own):
+def test_model_prompt_follows_the_rule(monkeypatch, rows, own):
     """Qwen2Model.forward launches luc_prompt_gemm once a layer where the rule
     says so, and not at all elsewhere."""
     cfg = dataclasses.replace(model.QWEN25_05B, hidden_size=128, intermediate_size=128,
                               num_attention_heads=2, num_key_value_heads=1, num_hidden_layers=2,
                               vocab_size=64)
+    monkeypatch.setattr(model, "PROMPT_KERNEL_FEW", 0)
     lib = _NoLaunch()
     calls = []
     lib.prompt_gemm = lambda *a: calls.append(a[1].shape[0])

@@ -652,8 +652,8 @@ def test_prompt_products_agree_with_library_gemms(luc, monkeypatch, inter):
     w = random_weights(cfg, 5, std=0.06)
     ids = [int(i) for i in np.random.default_rng(6).integers(0, 512, 130)]
     got = []
-    for rows in (model_module.PROMPT_KERNEL_ROWS, 0):
-        monkeypatch.setattr(model_module, "PROMPT_KERNEL_ROWS", rows)
+    for own in (True, False):
+        monkeypatch.setattr(model_module, "prompt_kernels_win", lambda cfg, rows, own=own: own)
         m = Qwen2Model(cfg, w, max_positions=256, lib=luc)
         m.forward(ids, 0)
         got.append([t.float() for t in (m.hidden, m.logits(), m.kv.k_pool, m.kv.v_pool)])
